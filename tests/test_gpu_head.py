@@ -217,6 +217,22 @@ def test_folded_head_matches_oracle_bits(hs, name, H, block, signed):
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("H,block", [(16384, 2), (24576, 8192), (20480, 4096), (8192 + 32, 32), (8192 + 8, 8),
+                                     (128, 128), (12, 4), (4, 4), (6, 1)])
+def test_folded_rows_across_pieces(hs, H, block):
+    """The norm-and-fold kernel at the edges of its 8192-element pieces, with
+    fold blocks that take one, two and three stages at a time."""
+    rng = np.random.default_rng(H + block)
+    h = rng.normal(0, 2.0, (3, H)).astype(np.float32)
+    g = rng.normal(1.0, 0.2, H).astype(np.float32)
+    s = np.where(rng.random(H) < 0.5, -1.0, 1.0).astype(np.float32)
+    w = rng.normal(0, 0.04, (65, H)).astype(np.float32)
+    got, normed = _qhead(hs, h, g, w, O.HEAD_F32, 1.0, fold_block=block, signs=s)
+    want, want_n = O.lm_head(h, g, 1e-6, w, 1.0, dtype=O.HEAD_F32, fold_block=block, fold_signs=s)
+    np.testing.assert_array_equal(normed, want_n)
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_quant_head_feeds_the_sampler(hs, sampler, wl):
     """A Q6_K head's device logits sampled on the device: the oracle's tokens."""
     import torch

@@ -578,35 +578,107 @@ hipError_t launch_q(const ultima_hsamp_head* h, const float* xin, int64_t rb, bo
 // ---- the norm and the fold -------------------------------------------------------
 
 constexpr int kPrepThreads = 1024;
+constexpr int kPrepPiece = ULTIMA_HSAMP_MAX_FOLD_BLOCK;      // elements of a row in LDS at a time
+constexpr int kPrepPer = kPrepPiece / kPrepThreads;          // a thread's share of a piece
+constexpr int kPrepChain = kPrepPiece / 8 + 8;               // LDS floats of one chain (8 mod 64: conflict-free)
 
-// One block per batch row. The sum of squares' eight chains run on eight
-// threads of wave 0 (the reference's order: chain l over elements l, l + 8,
-// ...); the normed row goes to LDS when a fold follows (one fold block at a
-// time), else straight out.
+// 2^R butterfly inputs `len` apart in registers: the stages len, 2 len, .. of
+// the fold, the same additions on the same values as one stage at a time.
+template <int R>
+__device__ __forceinline__ void fold_stages(float* buf, int len, int n) {
+    constexpr int N = 1 << R;
+    auto at = [](int i) { return i + (i >> 3); };            // padded: every stride used below is conflict-free
+    for (int p = threadIdx.x; p < n / N; p += kPrepThreads) {
+        const int j = (p / len) * N * len + (p % len);
+        float v[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = buf[at(j + e * len)];
+#pragma unroll
+        for (int h = 1; h < N; h <<= 1)
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+                if ((e & h) == 0) {
+                    const float a = v[e], b = v[e + h];
+                    v[e] = a + b;
+                    v[e + h] = a - b;
+                }
+#pragma unroll
+        for (int e = 0; e < N; ++e) buf[at(j + e * len)] = v[e];
+    }
+    __syncthreads();
+}
+
+// One block per batch row; bound by the sum of squares' serial order (eight
+// chains of H / 8 dependent multiply-adds, ~1.7 us at H = 4096) and three
+// round trips to memory. The row comes in pieces of 8192 elements: coalesced
+// loads by every thread, stored chain-major in LDS, from which eight lanes
+// run the chains, four steps per 16-byte read and the next sixteen steps' reads
+// in flight. A fold takes all the fold blocks of a piece at once, three of its
+// stages per barrier in registers. H = 4096, one row: 29.3 -> 5.9 us (the
+// chains read global memory eight elements at a time before); sixteen rows
+// with a 128-block fold: 95.6 -> 9.1 us (a barrier per stage of each fold
+// block before).
 __global__ __launch_bounds__(kPrepThreads) void k_head_prep(const float* __restrict__ hidden, int64_t hstride,
                                                             const float* __restrict__ scale, float eps, int H,
                                                             int fold_block, const float* __restrict__ signs,
                                                             float* __restrict__ normed) {
     __shared__ float red[8];
-    __shared__ float buf[ULTIMA_HSAMP_MAX_FOLD_BLOCK];
+    __shared__ __attribute__((aligned(16))) float buf[kPrepPiece + kPrepPiece / 8];
+    static_assert(8 * kPrepChain <= kPrepPiece + kPrepPiece / 8, "the chains fit the fold's buffer");
     const int row = blockIdx.x;
     const float* x = hidden + (int64_t)row * hstride;
     float* y = normed + (int64_t)row * H;
     const int tid = threadIdx.x;
     const int H8 = H / 8 * 8;
-    if (tid < 8) {
-        float p = 0.0f;
-        int k = tid;
-        for (; k + 8 * 7 < H8; k += 64) {
-            float v[8];
+    const bool fold = fold_block > 0 && H % fold_block == 0;
+    // a piece's elements, scales and signs; indices clamped into the row
+    float pv[kPrepPer], sv[kPrepPer], gv[kPrepPer];
+    auto load = [&](int p0, float* v, const float* from) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = x[k + 8 * e];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) p = __builtin_fmaf(v[e], v[e], p);
+        for (int e = 0; e < kPrepPer; ++e) v[e] = from[min(p0 + tid + e * kPrepThreads, H - 1)];
+    };
+    load(0, pv, x);
+    load(0, sv, scale);
+    if (fold && signs != nullptr) load(0, gv, signs);
+    float p = 0.0f;
+    for (int p0 = 0; p0 < H8; p0 += kPrepPiece) {
+        if (p0 > 0) {
+            load(p0, pv, x);
+            __syncthreads();                                 // the previous piece's chains are done
         }
-        for (; k < H8; k += 8) p = __builtin_fmaf(x[k], x[k], p);
-        red[tid] = p;
+#pragma unroll
+        for (int e = 0; e < kPrepPer; ++e) {
+            const int k = tid + e * kPrepThreads;
+            buf[(k & 7) * kPrepChain + (k >> 3)] = pv[e];
+        }
+        __syncthreads();
+        if (tid < 8) {
+            const int n = min(kPrepPiece, H8 - p0) >> 3;     // steps of this piece
+            const float* cf = buf + tid * kPrepChain;
+            const float4* cs = reinterpret_cast<const float4*>(cf);
+            const int ng = n >> 4;
+            float4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = cs[i];
+            for (int g = 0; g < ng; ++g) {
+                float4 w[4];
+                const float4* nx = cs + 4 * min(g + 1, ng - 1);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = nx[i];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    p = __builtin_fmaf(v[i].x, v[i].x, p);
+                    p = __builtin_fmaf(v[i].y, v[i].y, p);
+                    p = __builtin_fmaf(v[i].z, v[i].z, p);
+                    p = __builtin_fmaf(v[i].w, v[i].w, p);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = w[i];
+            }
+            for (int j = 16 * ng; j < n; ++j) p = __builtin_fmaf(cf[j], cf[j], p);
+        }
     }
+    if (tid < 8) red[tid] = p;
     __syncthreads();
     float ss = hsum8(red);
     // the tail as GCC compiles the reference's vectorised loop: the first four
@@ -619,28 +691,41 @@ __global__ __launch_bounds__(kPrepThreads) void k_head_prep(const float* __restr
         for (; i < t; ++i) ss = __builtin_fmaf(x[H8 + i], x[H8 + i], ss);
     }
     const float inv = 1.0f / sqrtf(ss / (float)H + eps);
-    const bool fold = fold_block > 0 && H % fold_block == 0;
-    if (!fold) {
-        for (int i = tid; i < H; i += kPrepThreads) y[i] = (x[i] * scale[i]) * inv;
-        return;
-    }
     const float finv = 1.0f / sqrtf((float)fold_block);
-    for (int off = 0; off < H; off += fold_block) {
-        for (int i = tid; i < fold_block; i += kPrepThreads) {
-            const float v = (x[off + i] * scale[off + i]) * inv;
-            buf[i] = signs != nullptr ? v * signs[off + i] : v;
+    for (int p0 = 0; p0 < H; p0 += kPrepPiece) {
+        if (H > kPrepPiece) {                                // (one piece: still in registers)
+            load(p0, pv, x);
+            load(p0, sv, scale);
+            if (fold && signs != nullptr) load(p0, gv, signs);
+        }
+        const int n = min(kPrepPiece, H - p0);
+        if (!fold) {
+#pragma unroll
+            for (int e = 0; e < kPrepPer; ++e) {
+                const int i = tid + e * kPrepThreads;
+                if (i < n) y[p0 + i] = (pv[e] * sv[e]) * inv;
+            }
+            continue;
+        }
+        // (fold blocks are powers of two up to the piece: n is a whole number of them)
+#pragma unroll
+        for (int e = 0; e < kPrepPer; ++e) {
+            const int i = tid + e * kPrepThreads;
+            const float v = (pv[e] * sv[e]) * inv;
+            if (i < n) buf[i + (i >> 3)] = signs != nullptr ? v * gv[e] : v;
         }
         __syncthreads();
-        for (int len = 1; len < fold_block; len <<= 1) {
-            for (int p = tid; p < fold_block / 2; p += kPrepThreads) {
-                const int j = (p / len) * 2 * len + (p % len);
-                const float u = buf[j], v = buf[j + len];
-                buf[j] = u + v;
-                buf[j + len] = u - v;
-            }
-            __syncthreads();
+        for (int len = 1; len < fold_block;) {
+            const int left = fold_block / len;
+            if (left >= 8) fold_stages<3>(buf, len, n), len *= 8;
+            else if (left == 4) fold_stages<2>(buf, len, n), len *= 4;
+            else fold_stages<1>(buf, len, n), len *= 2;
         }
-        for (int i = tid; i < fold_block; i += kPrepThreads) y[off + i] = fold_block >= 2 ? buf[i] * finv : buf[i];
+#pragma unroll
+        for (int e = 0; e < kPrepPer; ++e) {
+            const int i = tid + e * kPrepThreads;
+            if (i < n) y[p0 + i] = fold_block >= 2 ? buf[i + (i >> 3)] * finv : buf[i + (i >> 3)];
+        }
         __syncthreads();
     }
 }
