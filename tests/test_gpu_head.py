@@ -55,6 +55,31 @@ def test_lm_head_matches_oracle_bits(hs, rows, H, V, dtype, scale):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,H,V", [
+    (5, 896, 301),       # the fewest rows of the matrix-core kernel: one tile of batch rows, a ragged vocabulary tile
+    (16, 256, 64),       # whole tiles and chunks
+    (17, 264, 65),       # two tiles, a step past the whole chunks
+    (33, 1030, 70),      # three tiles, unaligned rows, a six-element tail
+    (49, 137, 31),       # four tiles, rows at odd element addresses, a one-element tail
+    (64, 4096, 130),
+    (70, 36, 17),        # a second group of rows; fewer columns than a chunk, a four-element tail
+    (20, 8, 5), (9, 16, 3), (6, 24, 16), (6, 7, 20), (130, 72, 1),
+])
+def test_lm_head_many_rows_matches_oracle_bits(hs, rows, H, V, dtype):
+    rng = np.random.default_rng(rows * 1000 + H + V)
+    h = rng.normal(0, 2.0, (rows, H)).astype(np.float32)
+    g = rng.normal(1.0, 0.2, H).astype(np.float32)
+    w = rng.normal(0, 0.04, (V, H)).astype(np.float32)
+    w[rng.random((V, H)) < 0.1] = -0.0
+    if dtype == "bf16":
+        w = bf16_bits(w)
+    got, normed = _head(hs, h, g, w, 2.5)
+    want, want_n = O.lm_head(h, g, 1e-6, w, 2.5)
+    np.testing.assert_array_equal(normed, want_n)
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_lm_head_feeds_the_sampler(hs, sampler, wl):
     """Device hidden states -> device logits -> sampled tokens, no host round
     trip in between: equal to the oracle's tokens on the oracle's logits."""

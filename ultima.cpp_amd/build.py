@@ -65,6 +65,7 @@ def build_all() -> None:
         "hsamp_api.o": CSRC / "hsamp_api.cpp",
         "hsamp_head.o": CSRC / "hsamp_head.hip",
         "hsamp_headq.o": CSRC / "hsamp_headq.hip",
+        "hsamp_headm.o": CSRC / "hsamp_headm.hip",
         "hsamp_history.o": CSRC / "hsamp_history.hip",
         "hsamp_callers.o": CSRC / "hsamp_callers.hip",
     }

@@ -42,17 +42,6 @@ constexpr int kGRS = kGRowBytes + 16;         // LDS bytes per row of the gemv t
 
 __device__ __forceinline__ float bf16f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
-// acc + a(0) b(0) + ... + a(t-1) b(t-1) as the reference's vectorised f32 tail
-// (t < 8): when t >= 4 the first four products are rounded on their own.
-template <class A, class B>
-__device__ __forceinline__ float tail_f32(float acc, A a, B b, int t) {
-    int i = 0;
-    if (t >= 4)
-        for (; i < 4; ++i) acc = acc + a(i) * b(i);
-    for (; i < t; ++i) acc = __builtin_fmaf(a(i), b(i), acc);
-    return acc;
-}
-
 // The horizontal sum of the eight partials held by lanes 8g .. 8g + 7 (lane
 // 8g + l holds partial l); every lane of the group gets it.
 __device__ __forceinline__ float hsum8_lanes(float p) {
@@ -372,9 +361,10 @@ extern "C" int ultima_hsamp_lm_head(const ultima_hsamp_head* h, void* hip_stream
     }
     const int es = h->weight_dtype == ULTIMA_HSAMP_BF16 ? 2 : 4;
     const bool vec = (reinterpret_cast<uintptr_t>(h->weight) % 16 == 0) && (((int64_t)h->hidden_dim * es) % 16 == 0);
-    if (fold) {
+    if (fold || h->rows > kGemvRows) {
         e = launch_head_prep(h, s);
-        if (e == hipSuccess)
+        if (e == hipSuccess && h->rows > kGemvRows) e = launch_head_mm(h, s);
+        else if (e == hipSuccess)
             e = h->weight_dtype == ULTIMA_HSAMP_BF16 ? launch_gemv<true, true>(h, vec, s) : launch_gemv<false, true>(h, vec, s);
     } else {
         e = h->weight_dtype == ULTIMA_HSAMP_BF16 ? launch_gemv<true, false>(h, vec, s) : launch_gemv<false, false>(h, vec, s);
