@@ -161,6 +161,41 @@ def test_quant_head_matches_oracle_bits(hs, name, rows, H, V, scale, offset):
     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("name", QNAMES)
+@pytest.mark.parametrize("rows,H,V,offset", [
+    (5, 1024, 65, 0),       # the fewest rows of the matrix-core kernel, a ragged vocabulary tile
+    (16, 768, 130, 0),      # an odd number of super-blocks: a chunk's last block missing, rows on odd half-dwords
+    (17, 512, 40, 4),       # two batch tiles
+    (33, 256, 33, 2),       # three: four tiles, or two of two
+    (64, 2304, 20, 1),      # odd byte addresses
+    (70, 1280, 17, 0),      # five tiles
+    (7, 96, 200, 0), (7, 1056, 200, 2),   # last chunks of fewer blocks (types of 32-value blocks)
+])
+@pytest.mark.parametrize("special", [False, True])
+def test_quant_head_many_rows_matches_oracle_bits(hs, name, rows, H, V, offset, special):
+    """More than four rows; special: fp16 scales that are subnormal, zero,
+    negative, infinite and NaN among the blocks (NaN logits compared as NaN)."""
+    dt = O.HEAD_NAMES[name]
+    if H % WL.QUANT_BLOCKS[dt][0] or (special and rows > 16):
+        pytest.skip("not a whole number of blocks, or covered by fewer rows")
+    rng = np.random.default_rng(rows * 7 + H + V + dt)
+    h = rng.normal(0, 2.0, (rows, H)).astype(np.float32)
+    g = rng.normal(1.0, 0.2, H).astype(np.float32)
+    w = WL.quant_head(dt, V, H, seed=H + V + dt)
+    if special:
+        blocks = w.reshape(-1, WL.QUANT_BLOCKS[dt][1])
+        v = np.resize(np.array([0x0001, 0x03FF, 0x0000, 0x8000, 0xBC00, 0x7C00, 0xFC00, 0x7E00, 0x7C01], np.uint16),
+                      blocks[::3].shape[0])
+        f = WL.QUANT_BLOCKS[dt][2][0]
+        blocks[::3, f], blocks[::3, f + 1] = v & 0xFF, v >> 8
+    got, normed = _qhead(hs, h, g, w, dt, 2.5, offset=offset)
+    want, want_n = O.lm_head(h, g, 1e-6, w, 2.5, dtype=dt)
+    np.testing.assert_array_equal(normed, want_n)
+    nan = np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
 @pytest.mark.parametrize("name", ["q8_0", "q4_1", "q5_0", "pq2_0"])
 @pytest.mark.parametrize("H", [96, 1056, 384])
 def test_quant_head_partial_chunks(hs, name, H):
