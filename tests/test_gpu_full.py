@@ -60,6 +60,48 @@ def test_full_vocab_with_penalties_and_bf16(sampler, wl):
         assert compare_rows(w, g) == rows
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("V,hist,knobs", [
+    (151936, 600, dict(temperature=0.8, top_p=0.95, min_p=0.05, rep_penalty=1.1, repeat_last_n=600)),
+    (2047, 64, dict(temperature=1.1, rep_penalty=0.7, repeat_last_n=40, frequency_penalty=-0.3)),   # raising, one block
+    (2049, 1, dict(temperature=0.9, top_p=0.8, presence_penalty=0.5, repeat_last_n=8)),             # one id past a block
+    (6145, 2500, dict(temperature=0.7, min_p=0.02, rep_penalty=1.3, repeat_last_n=100, dry_multiplier=0.8,
+                      dry_last_n=2500, frequency_penalty=0.2)),                                     # three windows of ids
+    (511, 300, dict(temperature=1.0, top_p=0.99, dry_multiplier=0.5, dry_last_n=300, rep_penalty=1.2,
+                    repeat_last_n=300)),
+])
+def test_full_vocab_penalised_rows_over_many_blocks(sampler, wl, V, hist, knobs, dtype):
+    """Whole-vocabulary rows with penalties and logit bias, whose transform
+    counts the history window by window: ids at the windows' and blocks'
+    edges and outside the vocabulary, bans and boosts, a masked row, one row
+    of the batch without penalties."""
+    rows = 4
+    plist = [wl.identity_params(**knobs) for _ in range(rows)]
+    plist[2] = wl.identity_params(temperature=0.8, top_p=0.9)
+    w = _wl(wl, V, rows, plist, seed=V + hist, sigma=3.0, dtype=dtype, hist_len=hist)
+    edges = np.array([0, 511, 512, 2047, 2048, V - 1, V, -1, 0, 511], np.int64)
+    k = min(hist, edges.size)
+    w.hist[1, -k:] = edges[:k]
+    w.hist[3] = np.where(np.arange(hist) % 3 == 0, int(np.argmax(w.logits_f32()[3])), w.hist[3])
+    w.mask = np.full((rows, (V + 31) // 32), 0xFFFFFFFF, np.uint32)
+    w.mask[1, ::5] = 0x00FF00FF
+    bias = [{0: 2.0, V - 1: -np.inf, min(512, V - 2): 5.0}, None, None, {int(np.argmax(w.logits_f32()[3])): -4.0}]
+    for wb in ((False, True) if dtype == "f32" else (False,)):
+        g = run_gpu(sampler, w, bias=bias, writeback=wb, set_cap=V)
+        assert compare_rows(w, g, bias=bias, writeback=wb) == rows
+
+
+def test_full_vocab_penalised_row_of_many_steps(hs, wl):
+    """V above a million: windows of two 512-id steps, counted one at a time."""
+    V, rows = (1 << 20) + 700, 2
+    p = wl.identity_params(temperature=0.8, top_p=0.9, rep_penalty=1.2, repeat_last_n=500, frequency_penalty=0.3)
+    w = _wl(wl, V, rows, [p] * rows, seed=5, sigma=3.0, hist_len=500)
+    w.hist[0, :6] = [0, 511, 512, 1023, 1024, V - 1]
+    s = hs.Sampler(0, max_rows=rows, max_vocab=V)
+    assert compare_rows(w, run_gpu(s, w, set_cap=V)) == rows
+    s.close()
+
+
 def test_full_vocab_mixed_with_topk_and_greedy_rows(sampler, wl):
     V, rows = 12000, 6
     plist = [wl.identity_params(temperature=1.0, top_p=0.9),

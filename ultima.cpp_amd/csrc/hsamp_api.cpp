@@ -26,7 +26,7 @@ namespace hsamp {
 hipError_t launch_stream(const StreamArgs& a, int dtype, bool vec, bool pen_greedy, bool pen_sample, bool mask,
                          bool greedy_rows, bool sample_rows, int grid, hipStream_t stream);
 hipError_t launch_writeback(const StreamArgs& a, int grid, uint32_t lds, hipStream_t stream);
-hipError_t launch_full_pre(const StreamArgs& a, bool plain, bool tp, hipStream_t stream);
+hipError_t launch_full_pre(const StreamArgs& a, bool plain, bool tp, bool pen, hipStream_t stream);
 hipError_t launch_merge(const StreamArgs& a, hipStream_t stream);
 hipError_t launch_pick_l(const StreamArgs& a, hipStream_t stream);
 hipError_t launch_stream_ex(const StreamArgs& a, int dtype, bool vec, bool pen, bool mask, int tiles, bool lean, int grid,
@@ -152,7 +152,7 @@ uint32_t fbits(float f) {
 namespace hsamp {
 
 // RowPlans + DRY tables + bias into hs.blob; the reference's predicates in [].
-int build_blob(HostScratch& hs, const ultima_hsamp_batch* b, Built& out) {
+int build_blob(HostScratch& hs, const ultima_hsamp_batch* b, Built& out, bool pen_fpre) {
     const int B = b->rows, V = b->vocab;
     hs.plans.assign(B, RowPlan{});
     std::vector<float>& dry = hs.dry;
@@ -283,18 +283,20 @@ int build_blob(HostScratch& hs, const ultima_hsamp_batch* b, Built& out) {
                 fl |= RF_FULL;                                                    // top-k off
             }
             if (fl & RF_FULL) out.any_full = true;
-            // plain transform (no penalties, no bias, no top-k): the row's whole-row
-            // passes run over many blocks ahead of k_full
-            if ((fl & RF_FULL) && !(fl & (RF_TOPK | RF_REP | RF_DRY | RF_FP | RF_BIAS))) {
+            // no top-k: the row's transform and whole-row passes run over many
+            // blocks ahead of k_full
+            const bool pens = (fl & (RF_REP | RF_DRY | RF_FP | RF_BIAS)) != 0;
+            if ((fl & RF_FULL) && !(fl & RF_TOPK) && (pen_fpre || !pens)) {
                 fl |= RF_FPRE;
                 out.any_fpre = true;
+                if (pens) out.any_fpre_pen = true;
             }
             else out.any_topk = out.any_sample = true;
             if ((fl & RF_FULL) && !(fl & RF_FPRE)) out.any_full_gen = true;
             if (q.top_p < 1.0f && !(q.top_p <= 0.0f)) fl |= RF_TOPP;             // [270, 147]
             if (q.min_p > 0.0f) fl |= RF_MINP;                                    // [273, 168]
             if (fl & RF_FPRE) {
-                if (fl & (RF_TOPP | RF_MINP)) out.any_fpre_tp = true;
+                if (pens || (fl & (RF_TOPP | RF_MINP))) out.any_fpre_tp = true;
                 else out.any_fpre_plain = true;
             }
             P.top_p = q.top_p;
@@ -547,8 +549,8 @@ int plan_run(const DevCaps& dc, const ultima_hsamp_batch* b, const Built& bl, Ru
     rp.merge_lds = merge_lds;
     // scratch
     rp.cand_slots = (size_t)nblocks;
-    rp.cand_elems = (size_t)nblocks * (size_t)cand_cap;
-    rp.ovf_elems = (size_t)B * kMergeRound;
+    rp.cand_elems = bl.any_topk ? (size_t)nblocks * (size_t)cand_cap : 0;
+    rp.ovf_elems = bl.any_topk ? (size_t)B * kMergeRound : 0;
     rp.gtab_words = gtab ? (size_t)B * 2 * mhash : 0;
     rp.full_elems = bl.any_full ? (size_t)B * rp.full_stride : 0;
     {
@@ -650,7 +652,7 @@ int launch_run(const RunPlan& rp, const Built& bl, const ultima_hsamp_batch* b, 
         else if (rp.exact) HIP_TRY(launch_pick(a, rp.pick_nw, stream));
         else if (bl.any_topk) HIP_TRY(launch_merge(a, stream));
         if (bl.any_full) {
-            if (bl.any_fpre) HIP_TRY(launch_full_pre(a, bl.any_fpre_plain, bl.any_fpre_tp, stream));
+            if (bl.any_fpre) HIP_TRY(launch_full_pre(a, bl.any_fpre_plain, bl.any_fpre_tp, bl.any_fpre_pen, stream));
             if (bl.any_full_gen) HIP_TRY(launch_full(a, (uint32_t)rp.full_lds, stream));
         }
         if (rp.wb) HIP_TRY(launch_writeback(a, rp.grid, (uint32_t)rp.wb_lds, stream));

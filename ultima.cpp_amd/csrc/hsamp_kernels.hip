@@ -4175,12 +4175,12 @@ __device__ void full_exp(const float* fv, float* pv, float m, int nW, int G, Ful
 
 // ---- full-vocabulary rows, their whole-row passes over many blocks ------------------
 // k_full runs one block per row; a row of the batch has V ids. For its rows
-// with a plain transform (RF_FPRE: mask and temperature, no penalties, no
-// logit bias, no top-k), the passes over the whole row that need no
+// without a top-k (RF_FPRE), the passes over the whole row that need no
 // sequential order run first over B x nW waves, one index-order window
 // (512 G ids) per wave, in the layout k_full uses (fullv / fullp, windows of
 // full_stride), and leave per-window tables (FS_*) for it:
-//   k_fs_max: the transform into fullv (the row's -inf padding included),
+//   k_fs_max: the transform (mask, penalties and bias, temperature) into
+//             fullv (the row's -inf padding included),
 //             each window's maximum m_w, whether it held a NaN, how many ids
 //             it leaves in and its sum of exp(x - m_w) (fast exp; a
 //             prediction only);
@@ -4213,14 +4213,26 @@ __device__ __forceinline__ uint4* fs_lanes(const StreamArgs& a, int r) {
 // k_fs_* blocks: kFsWaves waves, one window each.
 constexpr int kFsWaves = 4;
 
-template <int DT>
+// Penalties and logit bias (PEN: some row has them) without a table of the
+// row: a block's four windows are 2048 ids at a time, so it counts the row's
+// history hits among them in LDS (a word per id, the penalty table's fields),
+// takes stages 1-4 of the ids that were hit once, one per thread, and the pass
+// over the logits reads the result where the word is set. Bound by the reads
+// of the history by each of the row's blocks (L2), three barriers.
+// V = 151936, 16 rows, 600 ids, top-p and min-p: the step FSPEN us against
+// 654 for one block per row with a hash table probed per logit.
+template <int DT, bool PEN>
 __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
+    __shared__ __attribute__((aligned(16))) uint32_t phit[PEN ? kFsWaves * kFWin : 4];   // table fields, 0: not hit
+    __shared__ __attribute__((aligned(16))) float pval[PEN ? kFsWaves * kFWin : 4];      // the hit ids' values
     const int nW = fs_windows(a);
-    const int gw = (int)blockIdx.x * kFsWaves + wave_id();
-    const int r = gw / nW, w = gw - r * nW;
-    if (r >= a.rows) return;
+    const int nb = (nW + kFsWaves - 1) / kFsWaves;         // blocks per row
+    const int r = (int)blockIdx.x / nb, w0 = ((int)blockIdx.x - r * nb) * kFsWaves;
+    const int w = w0 + wave_id();
     const RowPlan P = plan_of(a, r);
     if (!(P.flags & RF_FPRE)) return;
+    const bool pen = PEN && (P.flags & (RF_REP | RF_DRY | RF_FP | RF_BIAS)) != 0;
+    if (!pen && w >= nW) return;                           // (a block with penalties keeps all its waves)
     const int lane = lane_id(), V = a.vocab, G = a.full_g, WS = kFWin * G;
     float* fv = a.fullv + (size_t)r * a.full_stride;
     const char* rowp = static_cast<const char*>(a.logits) + (size_t)r * (size_t)a.logits_stride * (DT == 0 ? 4 : 2);
@@ -4230,7 +4242,57 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
     int cnt = 0;
     // 16-byte loads where the row is aligned and the step lies inside it
     const bool al = (reinterpret_cast<uintptr_t>(rowp) & 15u) == 0u;
+    // step g's ids of the block's windows among the history and the bias, and their values
+    auto penalties = [&](int g) {
+        constexpr int NT = 64 * kFsWaves, N = kFsWaves * kFWin;
+        const int tid = threadIdx.x;
+        __syncthreads();                                   // (the step before has been read)
+#pragma unroll
+        for (int i = 0; i < N / NT; ++i) phit[tid + i * NT] = 0u;
+        __syncthreads();
+        auto place = [&](int t) {                          // id t's word, -1 where it is another block's or step's
+            if (t < 0 || t >= V) return -1;
+            const uint32_t o = (uint32_t)(t - w0 * WS);
+            if (t < w0 * WS || o >= (uint32_t)(kFsWaves * WS)) return -1;
+            const uint32_t k = o / (uint32_t)WS, in = o - k * (uint32_t)WS;
+            return (int)(in / kFWin) == g ? (int)(k * kFWin + in % kFWin) : -1;
+        };
+        const int L = hist_len_of(a, P, r), p0 = L - P.scan_len;
+        const int32_t* h = a.hist + (int64_t)r * a.hist_stride;
+        for (int b = p0; b < L; b += 8 * NT) {
+            int32_t t[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) t[q] = h[min(b + q * NT + tid, L - 1)];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int p = b + q * NT + tid, e = p < L ? place(t[q]) : -1;
+                if (e < 0) continue;
+                const uint32_t add = (p >= L - P.dry_win ? 1u << HV_DRY_SHIFT : 0u) + (p >= L - P.fp_win ? 1u : 0u);
+                if (add) atomicAdd(&phit[e], add);
+                if (p >= L - P.rep_win) atomicOr(&phit[e], (uint32_t)HV_REP);
+            }
+        }
+        if (P.flags & RF_BIAS)
+            for (int j = tid; j < P.bias_cnt; j += NT) {
+                const int e = place(a.bias_ids[P.bias_off + j]);
+                if (e >= 0) atomicOr(&phit[e], (uint32_t)HV_BIAS);
+            }
+        __syncthreads();
+        for (int e = tid; e < N; e += NT) {
+            const uint32_t hv = phit[e];
+            if (hv == 0u) continue;
+            const int t = (w0 + e / kFWin) * WS + g * kFWin + e % kFWin;
+            float y = load_logit<DT>(rowp, t);
+            if (mrow != nullptr && !((mrow[t >> 5] >> (t & 31)) & 1u)) y = -__builtin_inff();
+            pval[e] = pen_value(y, t, hv, a, P);
+        }
+        __syncthreads();
+    };
     for (int g = 0; g < G; ++g) {
+        if (pen) {
+            penalties(g);
+            if (w >= nW) continue;
+        }
         const int i0 = w * WS + g * kFWin + lane * 8;
         float x[8];
         uint32_t mw = 0xFFFFFFFFu;
@@ -4254,6 +4316,16 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
             for (int j = 0; j < 8; ++j) x[j] = load_logit<DT>(rowp, min(i0 + j, V - 1));
         }
         if (mrow != nullptr) mw = mrow[min(i0, V - 1) >> 5];   // (eight ids share one mask word)
+        uint32_t hit[8];
+        float hx[8];
+        if (pen) {
+            const int e = wave_id() * kFWin + lane * 8;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                hit[j] = phit[e + j];
+                hx[j] = pval[e + j];
+            }
+        }
         float y[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -4262,6 +4334,7 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
             if (i < V) {
                 v = x[j];
                 if (!((mw >> (i & 31)) & 1u)) v = -__builtin_inff();
+                if (pen && hit[j] != 0u) v = hx[j];
                 v = v * P.inv_temp;
                 if (v != v) {
                     nanv = true;
@@ -4291,6 +4364,7 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
         dst[0] = make_float4(y[0], y[1], y[2], y[3]);
         dst[1] = make_float4(y[4], y[5], y[6], y[7]);
     }
+    if (w >= nW) return;
     const float mw = wave_max_f(mloc);
     float rel = mloc == -__builtin_inff() ? 0.0f : lsum * __expf(mloc - mw);
     rel = readlane_f(wave_tree_prefix_f(rel), 63);
@@ -4475,8 +4549,8 @@ __device__ __forceinline__ void wave_ids_ascending(uint32_t* ids, int n, const f
 
 // Full-vocabulary rows, one block of kFT threads per row. PRE: the
 // instantiations for the RF_FPRE rows (k_fs_* did the transform and left the
-// window tables; no penalties, logit bias or top-k), PLAIN among them for the
-// rows without top-p and min-p (the CLI's identity() + temperature: without
+// window tables; no top-k), PLAIN among them for the
+// rows without penalties, top-p and min-p (the CLI's identity() + temperature: without
 // those stages' code the kernel keeps its state in registers); the other one
 // for the remaining full rows.
 template <bool GT, bool PRE, bool PLAIN>
@@ -4488,7 +4562,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     if (r >= a.rows) return;
     const RowPlan P = plan_of(a, r);
     if (!(P.flags & RF_FULL) || PRE != ((P.flags & RF_FPRE) != 0)) return;
-    if (PRE && PLAIN != ((P.flags & (RF_TOPP | RF_MINP)) == 0)) return;
+    if (PRE && PLAIN != ((P.flags & (RF_TOPP | RF_MINP | RF_REP | RF_DRY | RF_FP | RF_BIAS)) == 0)) return;
     HSAMP_PHASE(12000 + r, 0);
     const int V = a.vocab, G = a.full_g;
     const int WS = kFWin * G;
@@ -4576,6 +4650,9 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     using BT = std::integral_constant<bool, true>;
     using BF = std::integral_constant<bool, false>;
     constexpr bool pre = PRE;
+    // the draw's window sums of p from the numerators' double sums (rows with
+    // penalties take them value by value, as without RF_FPRE)
+    const bool sums = PRE && (P.flags & (RF_REP | RF_DRY | RF_FP | RF_BIAS)) == 0;
     static_assert(kFMaxWin <= 2 * kFT, "two windows per thread");
     double sdr[2] = {0.0, 0.0};   // PRE: the draw's window sums of the numerators ...
     uint32_t cnr[2] = {0u, 0u};   // ... and counts (windows tid, tid + kFT)
@@ -5051,7 +5128,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                         wn = 0;
                     }
                 });
-                fresh = pre;
+                fresh = sums;
                 __syncthreads();
             }
             S = xs_value(exact_index_sum(pv, nW, G, f, st, keep, pre ? fs_lanes(a, r) : nullptr));
@@ -5104,7 +5181,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             const float inv = 1.0f / S;
             double* wq = reinterpret_cast<double*>(f.winA);   // [kFMaxWin] window sums of p, then prefixes
             uint32_t* wc = f.winEF;                            // [kFMaxWin] kept counts, then prefixes
-            if (pre && !touched && !(P.flags & (RF_TOPP | RF_MINP))) {
+            if (PRE && (PLAIN || sums) && !touched && !(P.flags & (RF_TOPP | RF_MINP))) {
                 // k_fs_* left each window's numerators summed in double and
                 // its count: the window sums of p are taken as fl(1/S) times
                 // those (within 2^-24 of the sums of fl(e fl(1/S)) relative,
@@ -5577,12 +5654,15 @@ hipError_t launch_merge(const StreamArgs& a, hipStream_t stream) {
 
 // The RF_FPRE rows: k_fs_max, k_fs_exp over B x nW waves, then
 // k_full's PRE instantiations (no penalty table in their LDS): PLAIN for the
-// rows without top-p and min-p (plain), the other for the rows with them (tp).
-hipError_t launch_full_pre(const StreamArgs& a, bool plain, bool tp, hipStream_t stream) {
+// rows without top-p, min-p and penalties (plain), the other for the rest (tp).
+// pen: some of them have penalties or a logit bias.
+hipError_t launch_full_pre(const StreamArgs& a, bool plain, bool tp, bool pen, hipStream_t stream) {
     const int nW = a.full_stride / (kFWin * a.full_g);
-    const dim3 g((unsigned)(((int64_t)a.rows * nW + kFsWaves - 1) / kFsWaves)), b(64 * kFsWaves);
-    if (a.dtype == 0) hipLaunchKernelGGL((k_fs_max<0>), g, b, 0, stream, a);
-    else hipLaunchKernelGGL((k_fs_max<1>), g, b, 0, stream, a);
+    const dim3 g((unsigned)((int64_t)a.rows * ((nW + kFsWaves - 1) / kFsWaves))), b(64 * kFsWaves);
+    if (a.dtype == 0 && pen) hipLaunchKernelGGL((k_fs_max<0, true>), g, b, 0, stream, a);
+    else if (a.dtype == 0) hipLaunchKernelGGL((k_fs_max<0, false>), g, b, 0, stream, a);
+    else if (pen) hipLaunchKernelGGL((k_fs_max<1, true>), g, b, 0, stream, a);
+    else hipLaunchKernelGGL((k_fs_max<1, false>), g, b, 0, stream, a);
     const int run = fs_run(a.rows, nW), nq = (nW + run - 1) / run;
     const dim3 ge((unsigned)(((int64_t)a.rows * nq + kFsWaves - 1) / kFsWaves));
     hipLaunchKernelGGL(k_fs_exp, ge, b, 0, stream, a);

@@ -138,36 +138,43 @@ extern "C" int ultima_hsamp_run_noalloc(const ultima_hsamp_batch* b, void* hip_s
 
     static thread_local HostScratch hs;
     Built bl;
-    st = build_blob(hs, b, bl);
-    if (st != ULTIMA_HSAMP_OK) return st;
     RunPlan rp;
-    st = plan_run(d->caps, b, bl, rp);
-    if (st != ULTIMA_HSAMP_OK) return st;
-
+    RunBuffers buf;
     // The array's layout for this run: [plans' region][slice counts + bounds]
     // [candidate lists][overflow][penalty tables][fullv][fullp][k_fs_* tables][kept ids][kept counts]
-    size_t off = kPlanBytes;
-    auto take = [&](size_t bytes) -> unsigned char* {
-        unsigned char* p = d->ptr + off;
-        off = align256(off + bytes);
-        return p;
+    auto lay_out = [&](bool pen_fpre) -> int {
+        bl = Built{};
+        int s = build_blob(hs, b, bl, pen_fpre);
+        if (s != ULTIMA_HSAMP_OK) return s;
+        s = plan_run(d->caps, b, bl, rp);
+        if (s != ULTIMA_HSAMP_OK) return s;
+        size_t off = kPlanBytes;
+        auto take = [&](size_t bytes) -> unsigned char* {
+            unsigned char* p = d->ptr + off;
+            off = align256(off + bytes);
+            return p;
+        };
+        buf = RunBuffers{};
+        buf.cand_slots = rp.cand_slots;
+        buf.cand_n = reinterpret_cast<int32_t*>(take(rp.cand_slots * 8));
+        buf.cand = reinterpret_cast<unsigned long long*>(take(rp.cand_elems * 8));
+        buf.ovf = reinterpret_cast<unsigned long long*>(take(rp.ovf_elems * 8));
+        if (rp.gtab_words) buf.gtab = reinterpret_cast<uint32_t*>(take(rp.gtab_words * 4));
+        if (rp.full_elems) {
+            buf.fullv = reinterpret_cast<float*>(take(rp.full_elems * 4));
+            buf.fullp = reinterpret_cast<float*>(take(rp.full_elems * 4));
+        }
+        if (rp.fs_elems) buf.fs_tab = reinterpret_cast<uint32_t*>(take(rp.fs_elems * 4));
+        if (rp.fin_elems) {
+            buf.fin_idx = reinterpret_cast<int32_t*>(take(rp.fin_elems * 4));
+            buf.fin_n = reinterpret_cast<int32_t*>(take((size_t)rp.B * 4));
+        }
+        return off > kScratchBytes ? ULTIMA_HSAMP_ERR_CAPACITY : ULTIMA_HSAMP_OK;
     };
-    RunBuffers buf;
-    buf.cand_slots = rp.cand_slots;
-    buf.cand_n = reinterpret_cast<int32_t*>(take(rp.cand_slots * 8));
-    buf.cand = reinterpret_cast<unsigned long long*>(take(rp.cand_elems * 8));
-    buf.ovf = reinterpret_cast<unsigned long long*>(take(rp.ovf_elems * 8));
-    if (rp.gtab_words) buf.gtab = reinterpret_cast<uint32_t*>(take(rp.gtab_words * 4));
-    if (rp.full_elems) {
-        buf.fullv = reinterpret_cast<float*>(take(rp.full_elems * 4));
-        buf.fullp = reinterpret_cast<float*>(take(rp.full_elems * 4));
-    }
-    if (rp.fs_elems) buf.fs_tab = reinterpret_cast<uint32_t*>(take(rp.fs_elems * 4));
-    if (rp.fin_elems) {
-        buf.fin_idx = reinterpret_cast<int32_t*>(take(rp.fin_elems * 4));
-        buf.fin_n = reinterpret_cast<int32_t*>(take((size_t)rp.B * 4));
-    }
-    if (off > kScratchBytes) return ULTIMA_HSAMP_ERR_CAPACITY;
+    st = lay_out(true);
+    // rows with penalties need no window tables if they do not fit
+    if (st == ULTIMA_HSAMP_ERR_CAPACITY && bl.any_fpre_pen) st = lay_out(false);
+    if (st != ULTIMA_HSAMP_OK) return st;
 
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess) return hip_fail(hipErrorUnknown, "hipStreamIsCapturing", __LINE__);

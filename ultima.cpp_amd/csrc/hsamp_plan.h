@@ -33,8 +33,8 @@ enum : uint32_t {
     RF_FULL = 1u << 11,   // sampling row over the whole vocabulary: top-k off or above kLimitK (k_full)
     RF_DEVWIN = 1u << 12, // the row's history length is read on the device: the windows are taken
                           // there, min(cap, length), from the caps in RowPlan::win_caps
-    RF_FPRE = 1u << 13,   // a k_full row with a plain transform (no penalties, no logit bias, no
-                          // top-k): its whole-row passes run over many blocks first (k_fs_*)
+    RF_FPRE = 1u << 13,   // a k_full row without a top-k: its transform and whole-row passes run
+                          // over many blocks first (k_fs_*)
 };
 
 // k_fs_* per-row tables, nW entries each (nW = full_stride / (512 * full_g)):

@@ -60,10 +60,11 @@ struct Built {
     bool any_sample = false;   // a top-k sampling row (k_stream's sampling kernel)
     bool dry_split = false;    // a row whose DRY and frequency/presence windows differ
     bool two_windows = false;  // a row whose repetition and count windows are both on and differ
-    bool any_fpre = false;     // a k_full row with a plain transform (RF_FPRE)
+    bool any_fpre = false;     // a k_full row without a top-k (RF_FPRE)
+    bool any_fpre_pen = false; // ... with penalties or a logit bias
     bool any_full_gen = false; // a k_full row without RF_FPRE
-    bool any_fpre_plain = false;  // an RF_FPRE row without top-p and min-p
-    bool any_fpre_tp = false;     // an RF_FPRE row with top-p or min-p
+    bool any_fpre_plain = false;  // an RF_FPRE row without penalties, top-p and min-p
+    bool any_fpre_tp = false;     // an RF_FPRE row with some of them
 };
 
 // Kernel choice, slicing, LDS sizes and scratch sizes (in elements) of one run.
@@ -102,8 +103,10 @@ struct RunBuffers {
 
 // Argument checks of ultima_hsamp_run (limits: max_rows / max_vocab).
 int validate_batch(const ultima_hsamp_batch* b, int32_t max_rows, int32_t max_vocab);
-// RowPlans + DRY tables + bias entries into hs.blob.
-int build_blob(HostScratch& hs, const ultima_hsamp_batch* b, Built& out);
+// RowPlans + DRY tables + bias entries into hs.blob. pen_fpre: rows with
+// penalties take RF_FPRE too (whose window tables are 2 bytes of scratch an id;
+// without it k_full does their passes in one block).
+int build_blob(HostScratch& hs, const ultima_hsamp_batch* b, Built& out, bool pen_fpre = true);
 // Kernel choice and sizes (dc carries the diagnostics overrides).
 int plan_run(const DevCaps& dc, const ultima_hsamp_batch* b, const Built& bl, RunPlan& rp);
 // Launches the run's kernels on `stream` (nothing is allocated or copied).
