@@ -925,10 +925,13 @@ __device__ __attribute__((noinline)) void finalize_row(const StreamArgs& a, cons
             // sampler.cpp:178-182 / discrete_distribution: double sum S, q = p / S,
             // partial sums of q (cp[V-1] = 1), the first cp >= u. A tree prefix
             // of p over its tree total decides when every comparison that
-            // decides the token and the CDF_NEAR flag is clear of u by 2e-6
-            // (for <= 1024 terms the tree and the sequential sums, quotients
-            // and partial sums differ by < 1e-12); otherwise the reference's
-            // sequential sums on one thread.
+            // decides the token (a partial sum against u) and the CDF_NEAR flag
+            // (their distance against 1e-6) is clear by 1e-11 (for <= 1024
+            // terms the tree and the sequential sums, quotients and partial
+            // sums differ by < 1e-12); otherwise the reference's sequential
+            // sums on one thread, ~65 us for 1000 ids: with the margin at 2e-6
+            // one or two rows of a 1024-row batch took it and the batch waited
+            // for them (k_pick_l 121 us instead of 78).
             bool decided = false;
             if (single || !(u > 0.0)) {
                 if (tid == 0) {
@@ -971,10 +974,12 @@ __device__ __attribute__((noinline)) void finalize_row(const StreamArgs& a, cons
                     st.hbefore = before;
                 }
                 __syncthreads();
-                const bool clear = (h0 != INT32_MAX) ? (fabs(st.hat - u) > 2e-6 && fabs(st.hbefore - u) > 2e-6)
-                                                     : fabs(1.0 - u) > 2e-6;
-                if (clear) {
+                auto sure = [](double d) { return d > 1e-11 && fabs(d - 1e-6) > 1e-11; };
+                const bool found = h0 != INT32_MAX;
+                const double da = found ? fabs(st.hat - u) : fabs(1.0 - u), db = found ? fabs(st.hbefore - u) : da;
+                if (sure(da) && sure(db)) {
                     decided = true;
+                    if (fmin(da, db) <= 1e-6) rflags |= ROWF_CDF_NEAR;
                     __syncthreads();   // every thread has read st.tok / st.hat
                     if (tid == 0) {
                         st.tok = (h0 != INT32_MAX) ? f.fidx[h0] : V - 1;
