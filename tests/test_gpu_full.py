@@ -205,6 +205,34 @@ def test_plain_transform_rows_exact_sums(hs, sampler, wl, V):
     assert compare_rows(w, g) == rows
 
 
+@pytest.mark.parametrize("sigma,top_p,temp", [(3.0, 1.0, 0.8), (3.0, 0.95, 0.8), (0.5, 1.0, 1.0), (0.5, 0.9, 1.0),
+                                               (1.5, 0.999, 1.0), (6.0, 0.6, 1.0)])
+def test_min_p_at_a_numerators_edge(sampler, wl, sigma, top_p, temp):
+    """min_p set to one id's exp(x - max), a float above and a float below
+    (the ids the numerators alone do not decide), to 1 and above, to values
+    that remove nothing or all but a few ids, alone and after top-p, with
+    kept sets of one wave's list and of many thousands; two ids share the
+    largest logit. Rows with and without penalties."""
+    V = 20011
+    row = wl._rows_normal(int(sigma * 10), 1, V, sigma)[0]
+    row[7] = row[19000] = np.float32(row.max() + 0.25)
+    x = (row * np.float32(1.0 / np.float32(temp))) if temp != 1.0 else row
+    e = np.exp((x - x.max()).astype(np.float32).astype(np.float64)).astype(np.float32)
+    order = np.sort(e)[::-1]
+    edges = []
+    for k in (3, 300, 3000):
+        v = order[k]
+        edges += [v, np.nextafter(v, np.float32(2)), np.nextafter(v, np.float32(0))]
+    edges += [np.float32(1), np.float32(1.0000001), np.float32(2), np.float32(1e-25), np.float32(1e-12), np.float32(0.05)]
+    for pen in (False, True):
+        kw = dict(rep_penalty=1.3, repeat_last_n=32) if pen else {}
+        plist = [wl.identity_params(temperature=temp, top_p=top_p, min_p=float(v), **kw) for v in edges]
+        w = _wl(wl, V, len(edges), plist, seed=3, hist_len=32 if pen else 0)
+        w.logits[:] = row
+        g = run_gpu(sampler, w, writeback=pen, set_cap=V)
+        assert compare_rows(w, g, writeback=pen) == len(edges)
+
+
 def test_full_vocab_draw_without_sets(sampler, wl):
     """With no kept set asked for, rows whose top-p or min-p removed ids take
     the draw's window sums from the numerators alone and their kept count from

@@ -4799,6 +4799,9 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
         bool mk_same = true;    // the largest logit left in is still m
         int list_need = -1;     // top-p's candidates (p >= p*) fit one wave's list: the ids with p* it keeps
         uint32_t list_key = 0u; // ... and p*
+        // min-p can be decided on the numerators (below): a threshold of at
+        // most 1 and far from the subnormals, a finite maximum
+        const bool mpf = !PLAIN && (P.flags & RF_MINP) && P.min_p <= 1.0f && P.min_p >= 1e-20f && fabsf(m) < __builtin_inff();
 
         // ---- top-p (sampler.cpp:146-164) ----
         if (!PLAIN && (P.flags & RF_TOPP)) {
@@ -4823,14 +4826,16 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                 // the largest logit's p is fl(1 * inv) = inv: it stays in unless
                 // the cut falls among the ids with that p
                 if (cut_key == __float_as_uint(inv) && need < neq) mk_same = false;
-                if (!(P.flags & RF_MINP) && ngt + neq <= kFSort) {
+                // (min-p after it: on the list, or by the predicate below)
+                const bool pred = !(P.flags & RF_MINP) || (mpf && mk_same);
+                if (pred && ngt + neq <= kFSort) {
                     // few candidates: the list below keeps the lowest `need` ids with p*
                     keep = Keep{inv, cut_key, 0x7FFFFFFF};
                     list_need = need;
                     list_key = cut_key;
-                } else if (need >= neq && !(P.flags & RF_MINP)) {
+                } else if (pred && need >= neq) {
                     keep = Keep{inv, cut_key, 0x7FFFFFFF};
-                } else if (!(P.flags & RF_MINP) && mk_same && neq <= kFSort) {
+                } else if (pred && mk_same && neq <= kFSort) {
                     // the cut splits the ids with p* (not the top ones): the
                     // lowest `need` of them by id stay; their ids, gathered and
                     // sorted, give the predicate's id limit
@@ -4927,7 +4932,44 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             }
         }
 
-        // A small kept set (top-p's candidates, p >= p*, at most 512 ids): the
+        // ---- min-p (sampler.cpp:167-176) from the numerators, without the sum
+        // S' of what top-p left: an id leaves when fl(e fl(1/S')) <
+        // fl(min_p fl(1/S')) (the largest p is fl(1/S'): its e is 1). For
+        // e >= min_p that is never so (rounding is monotone), for
+        // e < min_p (1 - 2^-21) always (the products differ by more than two
+        // of their ulps); when an e lies between, the stage below takes S'.
+        // One pass and a predicate instead of the sum, a pass of writes and
+        // another sum.
+        bool mp_done = false;
+        if (!PLAIN && mpf && mk_same && list_need < 0) {
+            const float lo = P.min_p * (1.0f - 0x1p-21f);
+            int left = 0, amb = 0;
+            fpass(pv, Vp, [&](int i, float e) {
+                if (e >= P.min_p) left += keep(e, i) > 0.0f;
+                else amb += e >= lo;
+            });
+            left = fblock_sum_i(left, st);
+            amb = fblock_sum_i(amb, st);
+            mp_done = amb == 0;
+            // (top-p's predicate may be the tighter one: then no id leaves)
+            if (mp_done && (keep.key == 0u || P.min_p * keep.inv > __uint_as_float(keep.key))) {
+                if (nleft < 0) {
+                    int c = 0;
+                    if (pre) c = (int)(cnr[0] + cnr[1]);
+                    else fpass(fv, Vp, [&](int, float x) { c += x != -__builtin_inff(); });
+                    nleft = fblock_sum_i(c, st);
+                }
+                if (left != nleft) {
+                    keep = Keep{1.0f, __float_as_uint(P.min_p), 0x7FFFFFFF};
+                    nleft = left;
+                    changed = true;
+                    touched = true;
+                    if (left <= kFSort) list_need = left;   // (list_key 0: every one stays)
+                }
+            }
+        }
+
+        // A small kept set (the candidates of top-p, p >= p*, or min-p, at most 512 ids): the
         // candidates are gathered and sorted by id, the lowest `need` with p*
         // kept, and the rest is done on the list by wave 0 -- the largest kept
         // logit (and the numerators again when it is below m), the exact
@@ -5002,11 +5044,43 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                         ++kpos;
                     }
                 }
-                const int n = __builtin_amdgcn_readlane(kpos, 63);
+                int n = __builtin_amdgcn_readlane(kpos, 63);
                 wave_sync();
                 XState s2{-126, 0u};
                 chain_replay(s2, eb, n, __builtin_inff());
-                const float inv2 = 1.0f / xs_value(s2);
+                float inv2 = 1.0f / xs_value(s2);
+                if (!PLAIN && (P.flags & RF_MINP)) {
+                    // min-p on the list (its largest p is fl(1 * inv2))
+                    const float thr = P.min_p * inv2;
+                    bool k2[8];
+                    int c2 = 0;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const int q = lane * 8 + j;
+                        li_[j] = q < n ? ids[q] : 0u;
+                        le_[j] = q < n ? eb[q] : 0u;
+                        k2[j] = q < n && !(__uint_as_float(le_[j]) * inv2 < thr);
+                        c2 += k2[j];
+                    }
+                    const int i2 = wave_incl_sum_i(c2);
+                    const int n2 = __builtin_amdgcn_readlane(i2, 63);
+                    if (n2 != n) {
+                        int at = i2 - c2;
+                        wave_sync();
+#pragma unroll
+                        for (int j = 0; j < 8; ++j)
+                            if (k2[j]) {
+                                ids[at] = li_[j];
+                                eb[at] = le_[j];
+                                ++at;
+                            }
+                        n = n2;
+                        wave_sync();
+                        s2 = XState{-126, 0u};
+                        chain_replay(s2, eb, n, __builtin_inff());
+                        inv2 = 1.0f / xs_value(s2);
+                    }
+                }
                 // the draw (sampler.cpp:178-182): q = p / S_d over the kept ids in index order
                 float pq[8];
                 int32_t iq[8];
@@ -5139,8 +5213,8 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             S = xs_value(exact_index_sum(pv, nW, G, f, st, keep, pre ? fs_lanes(a, r) : nullptr));
         };
 
-        // ---- min-p (sampler.cpp:167-176) ----
-        if (!PLAIN && (P.flags & RF_MINP)) {
+        // ---- min-p (sampler.cpp:167-176), where the numerators alone did not decide it ----
+        if (!PLAIN && (P.flags & RF_MINP) && !mp_done && !listed) {
             if (changed) refresh();
             changed = false;
             const float inv = 1.0f / S;
@@ -5160,14 +5234,16 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                 // ids left in are those with p >= thr > 0 (a removed id's p is 0)
                 const float thr = P.min_p * inv;
                 int left = 0;
+                const Keep k0 = keep;   // (ids top-p's predicate left out leave the arrays too)
                 fpass(pv, Vp, [&](int i, float e) {
-                    if (e * inv < thr) {
+                    if (!(k0(e, i) * inv >= thr)) {
                         fv[i] = -__builtin_inff();
                         pv[i] = 0.0f;
                     } else {
                         ++left;
                     }
                 });
+                keep = kKeepAll;
                 left = fblock_sum_i(left, st);
                 changed = left != nleft;
                 nleft = left;
