@@ -25,7 +25,8 @@
 namespace hsamp {
 hipError_t launch_stream(const StreamArgs& a, int dtype, bool vec, bool pen_greedy, bool pen_sample, bool mask,
                          bool greedy_rows, bool sample_rows, int grid, hipStream_t stream);
-hipError_t launch_writeback(const StreamArgs& a, int grid, uint32_t lds, hipStream_t stream);
+hipError_t launch_writeback(const StreamArgs& a, hipStream_t stream);
+hipError_t launch_stage(const void* from, void* to, int n, hipStream_t stream);
 hipError_t launch_full_pre(const StreamArgs& a, bool plain, bool tp, bool pen, hipStream_t stream);
 hipError_t launch_merge(const StreamArgs& a, hipStream_t stream);
 hipError_t launch_pick_l(const StreamArgs& a, hipStream_t stream);
@@ -100,16 +101,12 @@ struct ultima_hsamp {
     // freed) until destroy, so that replaying an earlier graph stays valid.
     bool captured = false;
     std::vector<void*> retired;
-    // sample_host staging
-    float* d_row = nullptr;
-    float* h_row = nullptr;       // pinned
-    int32_t* d_hist = nullptr;
-    int32_t* h_hist = nullptr;    // pinned
-    size_t hist_cap = 0;
-    double* d_u = nullptr;
-    int32_t* d_tok = nullptr;
-    double* h_u = nullptr;        // pinned
-    int32_t* h_tok = nullptr;     // pinned
+    // sample_host staging, the same layout on both sides: [u, 64 bytes][the
+    // row, whole 64-byte lines][history]
+    char* h_stage = nullptr;      // pinned
+    char* d_stage = nullptr;
+    size_t stage_cap = 0;
+    int32_t* h_tok = nullptr;     // pinned; the kernels write the token here
 };
 
 namespace hsamp {
@@ -496,8 +493,7 @@ int plan_run(const DevCaps& dc, const ultima_hsamp_batch* b, const Built& bl, Ru
     if (fast) merge_lds = std::max(merge_lds, fast_lds);
     rp.fast = fast;
     rp.pen_flag = fast && pen_flag;
-    rp.wb_lds = (gtab ? 0 : 8 * (size_t)mhash) + 4 * (size_t)bitmap_words;
-    if (merge_lds + statik > dc.lds_limit || rp.wb_lds + statik > dc.lds_limit ||
+    if (merge_lds + statik > dc.lds_limit ||
         (bl.any_full && rp.full_lds + statik > dc.lds_limit))
         return ULTIMA_HSAMP_ERR_CAPACITY;
     const int nblocks = B * S;
@@ -542,8 +538,8 @@ int plan_run(const DevCaps& dc, const ultima_hsamp_batch* b, const Built& bl, Ru
         if (rp.lds_ex + statik > dc.lds_limit || pick_lds + statik > dc.lds_limit) exact = false;
         else merge_lds = pick_lds;
     }
-    // write-back after the exact lists: k_writeback rebuilds the rows' penalty
-    // tables in LDS (no merge kernel leaves a global one)
+    // (write-back of rows whose penalty tables are too large for LDS stays with
+    // the general kernels)
     if (rp.wb && gtab) exact = false;
     rp.exact = exact;
     rp.merge_lds = merge_lds;
@@ -620,6 +616,7 @@ int launch_run(const RunPlan& rp, const Built& bl, const ultima_hsamp_batch* b, 
     a.fullv = buf.fullv;
     a.fullp = buf.fullp;
     a.fs_tab = buf.fs_tab;
+    a.wb_out = bl.any_full ? nullptr : buf.wb_out;   // (k_full writes its row back in place)
     a.full_stride = rp.full_stride;
     a.full_g = rp.full_g;
     a.gtab = rp.gtab ? buf.gtab : nullptr;
@@ -655,7 +652,9 @@ int launch_run(const RunPlan& rp, const Built& bl, const ultima_hsamp_batch* b, 
             if (bl.any_fpre) HIP_TRY(launch_full_pre(a, bl.any_fpre_plain, bl.any_fpre_tp, bl.any_fpre_pen, stream));
             if (bl.any_full_gen) HIP_TRY(launch_full(a, (uint32_t)rp.full_lds, stream));
         }
-        if (rp.wb) HIP_TRY(launch_writeback(a, rp.grid, (uint32_t)rp.wb_lds, stream));
+        if (rp.wb) HIP_TRY(launch_writeback(a, stream));
+        if (buf.wb_out != nullptr && bl.any_full)
+            HIP_TRY(launch_stage(b->logits, buf.wb_out, (rp.V + 3) / 4, stream));
     }
     return ULTIMA_HSAMP_OK;
 }
@@ -727,6 +726,22 @@ int grow(ultima_hsamp* h, bool capturing, T*& ptr, size_t& have, size_t need) {
         return ULTIMA_HSAMP_ERR_NOMEM;
     }
     have = need;
+    return ULTIMA_HSAMP_OK;
+}
+
+// sample_host's staging of V logits and L history ids, and the offset of the history
+size_t stage_hist(int32_t V) { return 64 + (((size_t)V * 4 + 63) & ~size_t(63)); }
+size_t stage_bytes(int32_t V, size_t L) { return (stage_hist(V) + L * 4 + 63) & ~size_t(63); }
+int grow_stage(ultima_hsamp* h, size_t n) {
+    if (n <= h->stage_cap) return ULTIMA_HSAMP_OK;
+    if (h->d_stage) HIP_TRY(hipFree(h->d_stage));
+    if (h->h_stage) HIP_TRY(hipHostFree(h->h_stage));
+    h->d_stage = nullptr;
+    h->h_stage = nullptr;
+    h->stage_cap = 0;
+    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&h->d_stage), n));
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&h->h_stage), n, hipHostMallocDefault));
+    h->stage_cap = n;
     return ULTIMA_HSAMP_OK;
 }
 
@@ -842,13 +857,8 @@ int ultima_hsamp_create(int device, int32_t max_rows, int32_t max_vocab, ultima_
     h->cand_slots = blocks;
     CREATE_TRY(hipMalloc(reinterpret_cast<void**>(&h->fin_idx), (size_t)max_rows * kLimitK * 4));
     CREATE_TRY(hipMalloc(reinterpret_cast<void**>(&h->fin_n), (size_t)max_rows * 4));
-    CREATE_TRY(hipMalloc(reinterpret_cast<void**>(&h->d_row), (size_t)max_vocab * 4 + 64));
-    CREATE_TRY(hipHostMalloc(reinterpret_cast<void**>(&h->h_row), (size_t)max_vocab * 4 + 64,
-                             hipHostMallocDefault));
-    CREATE_TRY(hipMalloc(reinterpret_cast<void**>(&h->d_u), 64));
-    CREATE_TRY(hipMalloc(reinterpret_cast<void**>(&h->d_tok), 64));
-    CREATE_TRY(hipHostMalloc(reinterpret_cast<void**>(&h->h_u), 64, hipHostMallocDefault));
     CREATE_TRY(hipHostMalloc(reinterpret_cast<void**>(&h->h_tok), 64, hipHostMallocDefault));
+    if (grow_stage(h, stage_bytes(max_vocab, 1024)) != ULTIMA_HSAMP_OK) return fail(ULTIMA_HSAMP_ERR_NOMEM);
     CREATE_TRY(hipDeviceSynchronize());
 #undef CREATE_TRY
     *out = h;
@@ -867,10 +877,10 @@ int ultima_hsamp_destroy(ultima_hsamp* h) {
     for (void* p : {(void*)h->ovf, (void*)h->cand, (void*)h->cand_n,
                     (void*)h->gtab, (void*)h->fullv, (void*)h->fullp, (void*)h->fs_tab,
                     (void*)h->fin_idx,
-                    (void*)h->fin_n, (void*)h->d_row, (void*)h->d_hist, (void*)h->d_u, (void*)h->d_tok})
+                    (void*)h->fin_n, (void*)h->d_stage})
         if (p) (void)hipFree(p);
     for (void* p : h->retired) (void)hipFree(p);
-    for (void* p : {(void*)h->h_row, (void*)h->h_hist, (void*)h->h_u, (void*)h->h_tok})
+    for (void* p : {(void*)h->h_stage, (void*)h->h_tok})
         if (p) (void)hipHostFree(p);
     if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
     (void)hipGetLastError();
@@ -879,11 +889,12 @@ int ultima_hsamp_destroy(ultima_hsamp* h) {
 }
 
 namespace {
-int run_impl(ultima_hsamp* h, const ultima_hsamp_batch* b, const ultima_hsamp_commit* commit, void* hip_stream);
+int run_impl(ultima_hsamp* h, const ultima_hsamp_batch* b, const ultima_hsamp_commit* commit, float* wb_out,
+             void* hip_stream);
 }
 
 int ultima_hsamp_run(ultima_hsamp* h, const ultima_hsamp_batch* b, void* hip_stream) {
-    return run_impl(h, b, nullptr, hip_stream);
+    return run_impl(h, b, nullptr, nullptr, hip_stream);
 }
 
 int ultima_hsamp_run_commit(ultima_hsamp* h, const ultima_hsamp_batch* b, const ultima_hsamp_commit* c,
@@ -894,11 +905,13 @@ int ultima_hsamp_run_commit(ultima_hsamp* h, const ultima_hsamp_batch* b, const 
         return ULTIMA_HSAMP_ERR_INVALID;
     if (c->n_stop < 0 || c->n_stop > 8 || (c->n_stop > 0 && c->stop_ids == nullptr)) return ULTIMA_HSAMP_ERR_INVALID;
     if (b != nullptr && (b->flags & ULTIMA_HSAMP_WRITEBACK)) return ULTIMA_HSAMP_ERR_UNSUPPORTED;
-    return run_impl(h, b, c, hip_stream);
+    return run_impl(h, b, c, nullptr, hip_stream);
 }
 
 namespace {
-int run_impl(ultima_hsamp* h, const ultima_hsamp_batch* b, const ultima_hsamp_commit* commit, void* hip_stream) {
+// wb_out: where the write-back of a one-row batch goes, in place of its logits
+int run_impl(ultima_hsamp* h, const ultima_hsamp_batch* b, const ultima_hsamp_commit* commit, float* wb_out,
+             void* hip_stream) {
     if (h == nullptr) return ULTIMA_HSAMP_ERR_INVALID;
     int st = validate_batch(b, h->max_rows, h->max_vocab);
     if (st != ULTIMA_HSAMP_OK) return st;
@@ -946,6 +959,7 @@ int run_impl(ultima_hsamp* h, const ultima_hsamp_batch* b, const ultima_hsamp_co
     buf.fin_n = h->fin_n;
     buf.blob = slot->dev;
     buf.commit = commit;
+    buf.wb_out = wb_out;
     st = launch_run(rp, bl, b, buf, stream, h->phase_ev);
     if (st != ULTIMA_HSAMP_OK) return st;
     if (!capturing) HIP_TRY(hipEventRecord(slot->ev, stream));
@@ -1009,27 +1023,20 @@ int ultima_hsamp_sample_host(ultima_hsamp* h, float* logits, int32_t vocab,
     if (vocab > h->max_vocab) return ULTIMA_HSAMP_ERR_CAPACITY;
     if (params->hist_len < 0 || (params->hist_len > 0 && hist == nullptr)) return ULTIMA_HSAMP_ERR_INVALID;
     HIP_TRY(hipSetDevice(h->device));
+    // The row, u and the history go through one pinned area, copied by a
+    // kernel of the stream; the kernels write the token and the row's
+    // write-back to pinned memory themselves. (Copies by the DMA engines wait
+    // for the kernels around them, and those for the copies, ~8 us each: five
+    // of them were half of a 156 us call at V = 151936, 92 us now.)
     hipStream_t s = h->own_stream;
-    const size_t L = (size_t)params->hist_len;
-    if (L > h->hist_cap) {
-        if (h->d_hist) HIP_TRY(hipFree(h->d_hist));
-        if (h->h_hist) HIP_TRY(hipHostFree(h->h_hist));
-        h->d_hist = nullptr;
-        h->h_hist = nullptr;
-        h->hist_cap = 0;
-        const size_t cap = std::max<size_t>(L, 1024);
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&h->d_hist), cap * 4));
-        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&h->h_hist), cap * 4, hipHostMallocDefault));
-        h->hist_cap = cap;
-    }
-    std::memcpy(h->h_row, logits, (size_t)vocab * 4);
-    HIP_TRY(hipMemcpyAsync(h->d_row, h->h_row, (size_t)vocab * 4, hipMemcpyHostToDevice, s));
-    if (L > 0) {
-        std::memcpy(h->h_hist, hist, L * 4);
-        HIP_TRY(hipMemcpyAsync(h->d_hist, h->h_hist, L * 4, hipMemcpyHostToDevice, s));
-    }
-    *h->h_u = u;
-    HIP_TRY(hipMemcpyAsync(h->d_u, h->h_u, 8, hipMemcpyHostToDevice, s));
+    const size_t L = (size_t)params->hist_len, n = stage_bytes(vocab, L);
+    int st = grow_stage(h, n);
+    if (st != ULTIMA_HSAMP_OK) return st;
+    float* h_row = reinterpret_cast<float*>(h->h_stage + 64);
+    std::memcpy(h->h_stage, &u, 8);
+    std::memcpy(h_row, logits, (size_t)vocab * 4);
+    if (L > 0) std::memcpy(h->h_stage + stage_hist(vocab), hist, L * 4);
+    HIP_TRY(launch_stage(h->h_stage, h->d_stage, (int)(n / 16), s));
     ultima_hsamp_params p = *params;
     p.bias_offset = 0;
     ultima_hsamp_batch b{};
@@ -1037,24 +1044,22 @@ int ultima_hsamp_sample_host(ultima_hsamp* h, float* logits, int32_t vocab,
     b.vocab = vocab;
     b.dtype = ULTIMA_HSAMP_F32;
     b.flags = writeback ? ULTIMA_HSAMP_WRITEBACK : 0u;
-    b.logits = h->d_row;
+    b.logits = h->d_stage + 64;
     b.logits_stride = ((int64_t)vocab + 3) & ~int64_t(3);
-    b.hist = L > 0 ? h->d_hist : nullptr;
+    b.hist = L > 0 ? reinterpret_cast<const int32_t*>(h->d_stage + stage_hist(vocab)) : nullptr;
     b.hist_stride = (int64_t)L;
-    b.u = h->d_u;
+    b.u = reinterpret_cast<const double*>(h->d_stage);
     b.params = &p;
     b.bias_ids = params->bias_count > 0 ? bias_ids + params->bias_offset : nullptr;
     b.bias_vals = params->bias_count > 0 ? bias_vals + params->bias_offset : nullptr;
-    b.token = h->d_tok;
-    int st = ultima_hsamp_run(h, &b, s);
+    b.token = h->h_tok;
+    st = run_impl(h, &b, nullptr, writeback ? h_row : nullptr, s);
     if (st != ULTIMA_HSAMP_OK) {
         (void)hipStreamSynchronize(s);
         return st;
     }
-    HIP_TRY(hipMemcpyAsync(h->h_tok, h->d_tok, 4, hipMemcpyDeviceToHost, s));
-    if (writeback) HIP_TRY(hipMemcpyAsync(h->h_row, h->d_row, (size_t)vocab * 4, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    if (writeback) std::memcpy(logits, h->h_row, (size_t)vocab * 4);
+    if (writeback) std::memcpy(logits, h_row, (size_t)vocab * 4);
     *token_out = *h->h_tok;
     return ULTIMA_HSAMP_OK;
 }

@@ -4088,62 +4088,102 @@ __global__ __launch_bounds__(kBlock, 4) void k_pick_l(StreamArgs a) {
     select_and_finalize(sa, sP, r, buf, f, st, rflags);
 }
 
-// ---- writeback -------------------------------------------------------------------
-
-template <bool GT>
-__global__ __launch_bounds__(kBlock) void k_writeback(StreamArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ StreamArgs sa;
-    __shared__ RowPlan sP;
+// ---- penalties of a range of ids -----------------------------------------------------
+// Stages 1-4 (bias, repetition, DRY, frequency/presence) for the ids of a
+// block's range without a table of the row: the history's hits among the N ids
+// counted in LDS (a word per id, the penalty table's fields), then the ids that
+// were hit taken once each, one per thread. place(t): id t's word or -1 when it
+// is not the range's; id(e): word e's id; val(t): id t's logit, masked. Leaves
+// phit[e] (0: not hit) and pval[e]; barriers before, between and after.
+template <int NT, int N, class Place, class Id, class Val>
+__device__ __forceinline__ void range_penalties(const StreamArgs& a, const RowPlan& P, int r, uint32_t* phit, float* pval,
+                                                Place place, Id id, Val val) {
     const int tid = threadIdx.x;
-    const int logical = (int)(blockIdx.x % kXcds) * a.blocks_per_xcd + (int)(blockIdx.x / kXcds);
-    const int r = div_slices(logical, a), s = logical - r * a.nslices;
-    if (r >= a.rows) return;
+    __syncthreads();                                       // (the words of a range before have been read)
+#pragma unroll
+    for (int i = 0; i < N / NT; ++i) phit[tid + i * NT] = 0u;
+    __syncthreads();
+    const int L = hist_len_of(a, P, r), p0 = L - P.scan_len;
+    const int32_t* h = a.hist + (int64_t)r * a.hist_stride;
+    for (int b = p0; b < L; b += 8 * NT) {
+        int32_t t[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t[q] = h[min(b + q * NT + tid, L - 1)];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int p = b + q * NT + tid, e = (p < L && t[q] >= 0 && t[q] < a.vocab) ? place(t[q]) : -1;
+            if (e < 0) continue;
+            const uint32_t add = (p >= L - P.dry_win ? 1u << HV_DRY_SHIFT : 0u) + (p >= L - P.fp_win ? 1u : 0u);
+            if (add) atomicAdd(&phit[e], add);
+            if (p >= L - P.rep_win) atomicOr(&phit[e], (uint32_t)HV_REP);
+        }
+    }
+    if (P.flags & RF_BIAS)
+        for (int j = tid; j < P.bias_cnt; j += NT) {
+            const int e = place(a.bias_ids[P.bias_off + j]);
+            if (e >= 0) atomicOr(&phit[e], (uint32_t)HV_BIAS);
+        }
+    __syncthreads();
+    for (int e = tid; e < N; e += NT) {
+        const uint32_t hv = phit[e];
+        if (hv != 0u) pval[e] = pen_value(val(id(e)), id(e), hv, a, P);
+    }
+    __syncthreads();
+}
+
+// ---- writeback -------------------------------------------------------------------
+// The state sample() leaves the logits in (sampler.cpp:235-265), in place or in
+// wb_out: a block per 2048 ids of a row, eight per thread in flight. Latency:
+// one row of V = 151936 took 35 us with a block per 8192-id slice, each
+// building the row's penalty table and loading one logit at a time; 16 us so, its
+// stores going to host memory.
+constexpr int kWbIds = 2048;
+
+__global__ __launch_bounds__(kBlock) void k_writeback(StreamArgs a) {
+    __shared__ uint32_t phit[kWbIds];
+    __shared__ float pval[kWbIds];
+    __shared__ uint32_t keepbm[kWbIds / 32];
+    const int tid = threadIdx.x, V = a.vocab;
+    const int nb = (V + kWbIds - 1) / kWbIds;
+    const int r = (int)blockIdx.x / nb, lo = ((int)blockIdx.x - r * nb) * kWbIds;
     const RowPlan P = plan_of(a, r);
     if (P.flags & RF_FULL) return;   // k_full writes its rows back itself
-    if (tid == 0) {
-        sa = a;
-        sP = P;
-    }
-    const int V = a.vocab;
-    const int lo = s * a.slice_len;
-    const int hi = min(V, lo + a.slice_len);
     const bool greedy = (P.flags & RF_GREEDY) != 0;
     const bool pen = (P.flags & (RF_REP | RF_DRY | RF_FP | RF_BIAS)) != 0;
-    // LDS: [row penalty table (when not global)] [kept ids of this slice]
-    const PenaltyLds pl = pen_table<GT>(a, r, smem);
-    uint32_t* keepbm = reinterpret_cast<uint32_t*>(smem) + (GT ? 0 : 2 * a.mhash_slots);
-    int32_t pre[8];
-    hist_prefetch(a, P, r, pen && !GT, pre);
-    for (int i = tid; i < a.bitmap_words; i += kBlock) keepbm[i] = 0u;
-    // a global table is the one k_merge built for this row; an LDS one is rebuilt
-    if (pen && !GT) pen_build_row(a, P, r, pl, pre);
-    else __syncthreads();
+    const float* row = static_cast<const float*>(a.logits) + (int64_t)r * a.logits_stride;
+    float* out = a.wb_out != nullptr ? a.wb_out : const_cast<float*>(row);
+    const uint32_t* mrow = (P.flags & RF_MASK) ? a.mask + (int64_t)r * a.mask_stride : nullptr;
+    auto masked = [&](float x, int t) {
+        return mrow != nullptr && !((mrow[t >> 5] >> (t & 31)) & 1u) ? -__builtin_inff() : x;
+    };
+    float x[kWbIds / kBlock];
+#pragma unroll
+    for (int q = 0; q < kWbIds / kBlock; ++q) x[q] = row[min(lo + q * kBlock + tid, V - 1)];
+    if (pen)
+        range_penalties<kBlock, kWbIds>(a, P, r, phit, pval,
+                                        [&](int t) { return (uint32_t)(t - lo) < (uint32_t)kWbIds ? t - lo : -1; },
+                                        [&](int e) { return lo + e; }, [&](int t) { return masked(row[t], t); });
     if (!greedy) {
+        if (tid < kWbIds / 32) keepbm[tid] = 0u;
+        __syncthreads();
         const int n = a.fin_n[r];
         for (int j = tid; j < n; j += kBlock) {
-            const int t = a.fin_idx[(int64_t)r * a.fin_cap + j];
-            if (t >= lo && t < hi) atomicOr(&keepbm[(t - lo) >> 5], 1u << ((t - lo) & 31));
+            const uint32_t o = (uint32_t)(a.fin_idx[(int64_t)r * a.fin_cap + j] - lo);
+            if (o < (uint32_t)kWbIds) atomicOr(&keepbm[o >> 5], 1u << (o & 31));
         }
         __syncthreads();
     }
-    float* row = static_cast<float*>(const_cast<void*>(a.logits)) + (int64_t)r * a.logits_stride;
-    const uint32_t* mrow = (P.flags & RF_MASK) ? a.mask + (int64_t)r * a.mask_stride : nullptr;
-    for (int e = lo + tid; e < hi; e += kBlock) {
-        float x = row[e];
-        if (mrow != nullptr && !((mrow[e >> 5] >> (e & 31)) & 1u)) x = -__builtin_inff();
-        if (pen) {
-            // ids without a table entry pass through unchanged
-            uint32_t sl = hslot(e, pl);
-            uint32_t hk;
-            while ((hk = tab_ld(&pl.hkey[sl])) != kEmpty && hk != (uint32_t)e) sl = (sl + 1) & pl.hmask;
-            if (hk == (uint32_t)e) x = pen_apply(x, e, sa, sP, pl);
-        }
+#pragma unroll
+    for (int q = 0; q < kWbIds / kBlock; ++q) {
+        const int o = q * kBlock + tid, t = lo + o;
+        if (t >= V) break;
+        float y = masked(x[q], t);
+        if (pen && phit[o] != 0u) y = pval[o];
         if (!greedy) {
-            if (P.flags & RF_TEMP) x = x * P.inv_temp;
-            if (!((keepbm[(e - lo) >> 5] >> ((e - lo) & 31)) & 1u)) x = -__builtin_inff();
+            if (P.flags & RF_TEMP) y = y * P.inv_temp;
+            if (!((keepbm[o >> 5] >> (o & 31)) & 1u)) y = -__builtin_inff();
         }
-        row[e] = x;
+        out[t] = y;
     }
 }
 
@@ -4218,14 +4258,11 @@ __device__ __forceinline__ uint4* fs_lanes(const StreamArgs& a, int r) {
 // k_fs_* blocks: kFsWaves waves, one window each.
 constexpr int kFsWaves = 4;
 
-// Penalties and logit bias (PEN: some row has them) without a table of the
-// row: a block's four windows are 2048 ids at a time, so it counts the row's
-// history hits among them in LDS (a word per id, the penalty table's fields),
-// takes stages 1-4 of the ids that were hit once, one per thread, and the pass
-// over the logits reads the result where the word is set. Bound by the reads
-// of the history by each of the row's blocks (L2), three barriers.
-// V = 151936, 16 rows, 600 ids, top-p and min-p: the step FSPEN us against
-// 654 for one block per row with a hash table probed per logit.
+// Penalties and logit bias (PEN: some row has them) by range_penalties over a
+// block's four windows, 2048 ids at a time: bound by the reads of the history
+// by each of the row's blocks (L2) and its barriers, 11 us for 16 rows of
+// V = 151936 with 600 ids; the step 205 us against 654 for one block per row
+// that probed a hash table per logit.
 template <int DT, bool PEN>
 __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
     __shared__ __attribute__((aligned(16))) uint32_t phit[PEN ? kFsWaves * kFWin : 4];   // table fields, 0: not hit
@@ -4247,51 +4284,21 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
     int cnt = 0;
     // 16-byte loads where the row is aligned and the step lies inside it
     const bool al = (reinterpret_cast<uintptr_t>(rowp) & 15u) == 0u;
-    // step g's ids of the block's windows among the history and the bias, and their values
+    // step g's ids of the block's windows
     auto penalties = [&](int g) {
-        constexpr int NT = 64 * kFsWaves, N = kFsWaves * kFWin;
-        const int tid = threadIdx.x;
-        __syncthreads();                                   // (the step before has been read)
-#pragma unroll
-        for (int i = 0; i < N / NT; ++i) phit[tid + i * NT] = 0u;
-        __syncthreads();
-        auto place = [&](int t) {                          // id t's word, -1 where it is another block's or step's
-            if (t < 0 || t >= V) return -1;
-            const uint32_t o = (uint32_t)(t - w0 * WS);
-            if (t < w0 * WS || o >= (uint32_t)(kFsWaves * WS)) return -1;
-            const uint32_t k = o / (uint32_t)WS, in = o - k * (uint32_t)WS;
-            return (int)(in / kFWin) == g ? (int)(k * kFWin + in % kFWin) : -1;
-        };
-        const int L = hist_len_of(a, P, r), p0 = L - P.scan_len;
-        const int32_t* h = a.hist + (int64_t)r * a.hist_stride;
-        for (int b = p0; b < L; b += 8 * NT) {
-            int32_t t[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) t[q] = h[min(b + q * NT + tid, L - 1)];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int p = b + q * NT + tid, e = p < L ? place(t[q]) : -1;
-                if (e < 0) continue;
-                const uint32_t add = (p >= L - P.dry_win ? 1u << HV_DRY_SHIFT : 0u) + (p >= L - P.fp_win ? 1u : 0u);
-                if (add) atomicAdd(&phit[e], add);
-                if (p >= L - P.rep_win) atomicOr(&phit[e], (uint32_t)HV_REP);
-            }
-        }
-        if (P.flags & RF_BIAS)
-            for (int j = tid; j < P.bias_cnt; j += NT) {
-                const int e = place(a.bias_ids[P.bias_off + j]);
-                if (e >= 0) atomicOr(&phit[e], (uint32_t)HV_BIAS);
-            }
-        __syncthreads();
-        for (int e = tid; e < N; e += NT) {
-            const uint32_t hv = phit[e];
-            if (hv == 0u) continue;
-            const int t = (w0 + e / kFWin) * WS + g * kFWin + e % kFWin;
-            float y = load_logit<DT>(rowp, t);
-            if (mrow != nullptr && !((mrow[t >> 5] >> (t & 31)) & 1u)) y = -__builtin_inff();
-            pval[e] = pen_value(y, t, hv, a, P);
-        }
-        __syncthreads();
+        range_penalties<64 * kFsWaves, kFsWaves * kFWin>(
+            a, P, r, phit, pval,
+            [&](int t) {
+                const uint32_t o = (uint32_t)(t - w0 * WS);
+                if (t < w0 * WS || o >= (uint32_t)(kFsWaves * WS)) return -1;
+                const uint32_t k = o / (uint32_t)WS, in = o - k * (uint32_t)WS;
+                return (int)(in / kFWin) == g ? (int)(k * kFWin + in % kFWin) : -1;
+            },
+            [&](int e) { return (w0 + e / kFWin) * WS + g * kFWin + e % kFWin; },
+            [&](int t) {
+                const float y = load_logit<DT>(rowp, t);
+                return mrow != nullptr && !((mrow[t >> 5] >> (t & 31)) & 1u) ? -__builtin_inff() : y;
+            });
     };
     for (int g = 0; g < G; ++g) {
         if (pen) {
@@ -5761,9 +5768,22 @@ hipError_t launch_full(const StreamArgs& a, uint32_t lds, hipStream_t stream) {
 
 size_t full_lds_bytes() { return kFullLdsBytes; }
 
-hipError_t launch_writeback(const StreamArgs& a, int grid, uint32_t lds, hipStream_t stream) {
-    if (a.gtab != nullptr) hipLaunchKernelGGL((k_writeback<true>), dim3(grid), dim3(kBlock), lds, stream, a);
-    else hipLaunchKernelGGL((k_writeback<false>), dim3(grid), dim3(kBlock), lds, stream, a);
+hipError_t launch_writeback(const StreamArgs& a, hipStream_t stream) {
+    const dim3 grid((unsigned)((int64_t)a.rows * ((a.vocab + kWbIds - 1) / kWbIds)));
+    hipLaunchKernelGGL(k_writeback, grid, dim3(kBlock), 0, stream, a);
+    return hipGetLastError();
+}
+
+// n 16-byte vectors between pinned host memory and the device, the whole range
+// in flight at once.
+__global__ __launch_bounds__(kBlock) void k_stage(const uint4* __restrict__ from, uint4* __restrict__ to, int n) {
+    const int i = (int)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) to[i] = from[i];
+}
+
+hipError_t launch_stage(const void* from, void* to, int n, hipStream_t stream) {
+    hipLaunchKernelGGL(k_stage, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, stream,
+                       static_cast<const uint4*>(from), static_cast<uint4*>(to), n);
     return hipGetLastError();
 }
 

@@ -151,6 +151,7 @@ struct StreamArgs {
     float* fullp;               // [rows * full_stride] k_full: softmax numerators
     int32_t full_stride;        // k_full: floats per row of fullv / fullp (whole windows of 512 * full_g)
     int32_t full_g;             // k_full: 512-id steps per index-order window
+    float* wb_out;              // k_writeback's output for the batch's one row (NULL: in place)
     uint32_t* fs_tab;           // [rows * FS_TABLES * nW] k_fs_* results for k_full's RF_FPRE rows, then
                                 // (16-byte aligned) [rows * nW * 64] uint4 lane tables
     uint32_t* gtab;             // [rows * 2 * mhash_slots] penalty tables, or NULL: tables in LDS

@@ -74,7 +74,7 @@ struct RunPlan {
     int ex_tiles = 1, grid = 0, full_stride = 0, full_g = 1;
     bool exact = false, vec = false, gtab = false, fast = false, pen_flag = false, wb = false;
     bool cnt_ranked = false;  // exact lists: history counts by rank (a bitmap over the slice)
-    size_t lds = 0, lds_ex = 0, merge_lds = 0, full_lds = 0, wb_lds = 0, cnt_bytes = 0, stage_off = 0;
+    size_t lds = 0, lds_ex = 0, merge_lds = 0, full_lds = 0, cnt_bytes = 0, stage_off = 0;
     // scratch the kernels use
     size_t cand_elems = 0;    // u64 candidate lists, B * S * cand_cap
     size_t cand_slots = 0;    // per-slice counts, then as many bounds (int32 each)
@@ -97,6 +97,8 @@ struct RunBuffers {
     uint32_t* fs_tab = nullptr;
     int32_t* fin_idx = nullptr;
     int32_t* fin_n = nullptr;
+    float* wb_out = nullptr;      // where one row's write-back ends up (device-visible, whole 16-byte
+                                  // vectors, as the row itself); null: in place
     const char* blob = nullptr;   // device copy of HostScratch::blob
     const ultima_hsamp_commit* commit = nullptr;   // ultima_hsamp_run_commit's rules, or none
 };
