@@ -54,8 +54,10 @@ __device__ __forceinline__ float hsum8_lanes(float p) {
     return __shfl(tot, lane_id() & ~7, 64);
 }
 
-// WB: bf16 weights (else f32). BB: batch rows per block (1, 2 or 4). VEC:
-// weight rows sit on 16-byte boundaries (16-byte loads; else element loads).
+// WB: bf16 weights (else f32). BB: batch rows per block (1, 2 or 4). NTL:
+// weights loaded past the caches (streamed_past). The 16-byte loads take any
+// alignment: rows of an odd H by element loads were half as fast (one row,
+// H = 2561, V = 100001 bf16: 235 -> 125 us).
 // PRE: `hidden` already holds the head's input (normed and folded by
 // k_head_prep): no norm here, the values are used as they are.
 // One wave per 64 vocabulary rows, lane i running the eight chains of row
@@ -66,7 +68,7 @@ __device__ __forceinline__ float hsum8_lanes(float p) {
 // time -- one step of all eight chains (bf16), or half a step (f32). The
 // normed rows' columns of the chunk go through LDS too and are read as
 // broadcasts. The block is the one wave: no barrier waits on another wave.
-template <bool WB, int BB, bool VEC, bool PRE>
+template <bool WB, int BB, bool NTL, bool PRE>
 __global__ __launch_bounds__(64) void k_head_gemv(const void* __restrict__ weight, int V, int H,
                                                   const float* __restrict__ hidden, int64_t hstride,
                                                   const float* __restrict__ scale, float eps,
@@ -107,16 +109,10 @@ __global__ __launch_bounds__(64) void k_head_gemv(const void* __restrict__ weigh
             const int v = lane + i * 64;
             const int m = min(m0 + (v >> 3), V - 1), col = c0 + (v & 7) * EPV;
             const W* rowp = wb + (int64_t)m * H;
-            if (VEC) {
-                typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-                const u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(rowp + min(col, H8 - EPV)));
-                reg[i] = make_uint4(t.x, t.y, t.z, t.w);
-            } else {
-                W e[EPV];
-#pragma unroll
-                for (int j = 0; j < EPV; ++j) e[j] = rowp[min(col + j, H8 - 1)];
-                reg[i] = *reinterpret_cast<const uint4*>(e);
-            }
+            typedef unsigned int u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+            const u32x4* from = reinterpret_cast<const u32x4*>(rowp + min(col, H8 - EPV));
+            const u32x4 t = NTL ? __builtin_nontemporal_load(from) : *from;
+            reg[i] = make_uint4(t.x, t.y, t.z, t.w);
         }
         const int k = min(c0 + lane, H8 - 1);
 #pragma unroll
@@ -302,14 +298,14 @@ __global__ __launch_bounds__(64) void k_head_gemv(const void* __restrict__ weigh
 }
 
 template <bool WB, int BB, bool PRE>
-hipError_t launch_gemv_bb(const ultima_hsamp_head* h, bool vec, hipStream_t s) {
+hipError_t launch_gemv_bb(const ultima_hsamp_head* h, bool ntl, hipStream_t s) {
     // one wave per 64 vocabulary rows: every wave the same work, all resident
     // at once for real vocabularies (151936 rows: 2374 waves)
     const dim3 grid((h->vocab + 63) / 64, (h->rows + BB - 1) / BB);
     // PRE: the head's input is the prepared rows in `normed`
     const float* in = PRE ? h->normed : h->hidden;
     const int64_t in_stride = PRE ? h->hidden_dim : h->hidden_stride;
-    if (vec)
+    if (ntl)
         hipLaunchKernelGGL((k_head_gemv<WB, BB, true, PRE>), grid, dim3(64), 0, s, h->weight, h->vocab, h->hidden_dim,
                            in, in_stride, h->norm_scale, h->eps, h->normed, h->rows,
                            h->logit_scale, h->logits, h->logits_stride);
@@ -320,12 +316,24 @@ hipError_t launch_gemv_bb(const ultima_hsamp_head* h, bool vec, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Non-temporal weight loads where the rows are aligned (misaligned loads share
+// their lines with their neighbours'), but for small heads of fewer waves than
+// SIMDs, which wait for each load: a stream that fills the chip, or that the
+// Infinity Cache holds little of, is faster past the caches (V = 151936,
+// H = 4096 208 against 230 us; V = 100000, H = 896 32.4 against 36.5; V = 50000,
+// H = 4096 73 against 81), V = 32000, H = 2048 through them (28.5 against 36.6).
+bool streamed_past(const ultima_hsamp_head* h, int es) {
+    const int64_t row = (int64_t)h->hidden_dim * es;
+    return reinterpret_cast<uintptr_t>(h->weight) % 16 == 0 && row % 16 == 0 &&
+           (h->vocab >= 64 * 1024 || row * h->vocab > (int64_t)128 << 20);
+}
+
 // batch rows per block: one weight pass per group of up to four rows
 template <bool WB, bool PRE>
-hipError_t launch_gemv(const ultima_hsamp_head* h, bool vec, hipStream_t s) {
-    if (h->rows == 1) return launch_gemv_bb<WB, 1, PRE>(h, vec, s);
-    if (h->rows == 2) return launch_gemv_bb<WB, 2, PRE>(h, vec, s);
-    return launch_gemv_bb<WB, 4, PRE>(h, vec, s);
+hipError_t launch_gemv(const ultima_hsamp_head* h, bool ntl, hipStream_t s) {
+    if (h->rows == 1) return launch_gemv_bb<WB, 1, PRE>(h, ntl, s);
+    if (h->rows == 2) return launch_gemv_bb<WB, 2, PRE>(h, ntl, s);
+    return launch_gemv_bb<WB, 4, PRE>(h, ntl, s);
 }
 
 }  // namespace
@@ -360,14 +368,14 @@ extern "C" int ultima_hsamp_lm_head(const ultima_hsamp_head* h, void* hip_stream
         return e == hipSuccess ? ULTIMA_HSAMP_OK : ULTIMA_HSAMP_ERR_HIP;
     }
     const int es = h->weight_dtype == ULTIMA_HSAMP_BF16 ? 2 : 4;
-    const bool vec = (reinterpret_cast<uintptr_t>(h->weight) % 16 == 0) && (((int64_t)h->hidden_dim * es) % 16 == 0);
+    const bool ntl = streamed_past(h, es);
     if (fold || h->rows > kGemvRows) {
         e = launch_head_prep(h, s);
         if (e == hipSuccess && h->rows > kGemvRows) e = launch_head_mm(h, s);
         else if (e == hipSuccess)
-            e = h->weight_dtype == ULTIMA_HSAMP_BF16 ? launch_gemv<true, true>(h, vec, s) : launch_gemv<false, true>(h, vec, s);
+            e = h->weight_dtype == ULTIMA_HSAMP_BF16 ? launch_gemv<true, true>(h, ntl, s) : launch_gemv<false, true>(h, ntl, s);
     } else {
-        e = h->weight_dtype == ULTIMA_HSAMP_BF16 ? launch_gemv<true, false>(h, vec, s) : launch_gemv<false, false>(h, vec, s);
+        e = h->weight_dtype == ULTIMA_HSAMP_BF16 ? launch_gemv<true, false>(h, ntl, s) : launch_gemv<false, false>(h, ntl, s);
     }
     return e == hipSuccess ? ULTIMA_HSAMP_OK : ULTIMA_HSAMP_ERR_HIP;
 }
