@@ -102,6 +102,27 @@ def test_full_vocab_penalised_row_of_many_steps(hs, wl):
     s.close()
 
 
+@pytest.mark.parametrize("V,dtype,align", [(8, "f32", 4), (15, "bf16", 8), (515, "f32", 4), (2053, "bf16", 8),
+                                           (4099, "f32", None), (151936, "bf16", None)])
+def test_top_p_rows_read_from_the_logits(sampler, wl, V, dtype, align):
+    """Batches whose rows all have a top-p or min-p and no penalties: no
+    transformed copy of an aligned row is kept, its values are taken from the
+    logits -- at ragged ends, with a mask and NaN logits beside them, ties that
+    top-p splits, and the write-back (align None: a misaligned or whole row)."""
+    rows = 4
+    plist = [wl.identity_params(temperature=t, **k) for t, k in
+             [(0.8, dict(top_p=0.9)), (1.3, dict(min_p=0.1)), (1.0, dict(top_p=0.5, min_p=0.01)), (0.7, dict(top_p=0.99))]]
+    w = _wl(wl, V, rows, plist, seed=V, sigma=2.0, dtype=dtype)
+    x = w.logits_f32().copy()
+    x[2] = np.float32(0.5)                     # one value: every cut splits a tie
+    w.logits = x if dtype == "f32" else wl.to_bf16_bits(x)
+    w.mask = np.full((rows, (V + 31) // 32), 0xFFFFFFFF, np.uint32)
+    w.mask[3, ::2] = 0x0FF0F0F1
+    for wb in ((False, True) if dtype == "f32" else (False,)):
+        g = run_gpu(sampler, w, writeback=wb, set_cap=V, row_align=align)
+        assert compare_rows(w, g, writeback=wb) == rows
+
+
 def test_full_vocab_mixed_with_topk_and_greedy_rows(sampler, wl):
     V, rows = 12000, 6
     plist = [wl.identity_params(temperature=1.0, top_p=0.9),

@@ -4225,7 +4225,7 @@ __device__ void full_exp(const float* fv, float* pv, float m, int nW, int G, Ful
 // (512 G ids) per wave, in the layout k_full uses (fullv / fullp, windows of
 // full_stride), and leave per-window tables (FS_*) for it:
 //   k_fs_max: the transform (mask, penalties and bias, temperature) into
-//             fullv (the row's -inf padding included),
+//             fullv (the row's -inf padding included; fs_lazy: not written),
 //             each window's maximum m_w, whether it held a NaN, how many ids
 //             it leaves in and its sum of exp(x - m_w) (fast exp; a
 //             prediction only);
@@ -4257,6 +4257,30 @@ __device__ __forceinline__ uint4* fs_lanes(const StreamArgs& a, int r) {
 
 // k_fs_* blocks: kFsWaves waves, one window each.
 constexpr int kFsWaves = 4;
+
+// Logits i0 .. i0 + 7 of a 16-byte aligned row, all of them ids below V, and a
+// logit's value after mask and temperature (a NaN counts as -inf).
+template <int DT>
+__device__ __forceinline__ void load8(const char* rowp, int i0, float (&x)[8]) {
+    if (DT == 0) {
+        const float4 c0 = reinterpret_cast<const float4*>(rowp + (size_t)i0 * 4)[0];
+        const float4 c1 = reinterpret_cast<const float4*>(rowp + (size_t)i0 * 4)[1];
+        x[0] = c0.x; x[1] = c0.y; x[2] = c0.z; x[3] = c0.w;
+        x[4] = c1.x; x[5] = c1.y; x[6] = c1.z; x[7] = c1.w;
+    } else {
+        const uint4 c = *reinterpret_cast<const uint4*>(rowp + (size_t)i0 * 2);
+        const uint32_t h[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x[2 * j] = __uint_as_float(h[j] << 16);
+            x[2 * j + 1] = __uint_as_float(h[j] & 0xFFFF0000u);
+        }
+    }
+}
+__device__ __forceinline__ float plain_value(float x, bool allowed, float inv_temp) {
+    const float v = (allowed ? x : -__builtin_inff()) * inv_temp;
+    return v != v ? -__builtin_inff() : v;
+}
 
 // Penalties and logit bias (PEN: some row has them) by range_penalties over a
 // block's four windows, 2048 ids at a time: bound by the reads of the history
@@ -4309,20 +4333,7 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
         float x[8];
         uint32_t mw = 0xFFFFFFFFu;
         if (al && w * WS + (g + 1) * kFWin <= V) {
-            if (DT == 0) {
-                const float4 c0 = reinterpret_cast<const float4*>(rowp + (size_t)i0 * 4)[0];
-                const float4 c1 = reinterpret_cast<const float4*>(rowp + (size_t)i0 * 4)[1];
-                x[0] = c0.x; x[1] = c0.y; x[2] = c0.z; x[3] = c0.w;
-                x[4] = c1.x; x[5] = c1.y; x[6] = c1.z; x[7] = c1.w;
-            } else {
-                const uint4 c = *reinterpret_cast<const uint4*>(rowp + (size_t)i0 * 2);
-                const uint32_t h[4] = {c.x, c.y, c.z, c.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    x[2 * j] = __uint_as_float(h[j] << 16);
-                    x[2 * j + 1] = __uint_as_float(h[j] & 0xFFFF0000u);
-                }
-            }
+            load8<DT>(rowp, i0, x);
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[j] = load_logit<DT>(rowp, min(i0 + j, V - 1));
@@ -4372,9 +4383,11 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
                 lsum += s8 * __expf(sm - mloc);
             }
         }
-        float4* dst = reinterpret_cast<float4*>(fv + i0);
-        dst[0] = make_float4(y[0], y[1], y[2], y[3]);
-        dst[1] = make_float4(y[4], y[5], y[6], y[7]);
+        if (!a.fs_lazy) {
+            float4* dst = reinterpret_cast<float4*>(fv + i0);
+            dst[0] = make_float4(y[0], y[1], y[2], y[3]);
+            dst[1] = make_float4(y[4], y[5], y[6], y[7]);
+        }
     }
     if (w >= nW) return;
     const float mw = wave_max_f(mloc);
@@ -4400,6 +4413,9 @@ __host__ __device__ __forceinline__ int fs_run(int rows, int nW) {
     return (int64_t)rows * nW >= 16384 ? 4 : 1;
 }
 
+// LAZY (a.fs_lazy): the transformed values from the logits themselves (DT, their
+// type), not from fullv, which k_fs_max has not written.
+template <bool LAZY, int DT>
 __global__ __launch_bounds__(64 * kFsWaves) void k_fs_exp(StreamArgs a) {
     __shared__ uint64_t expT[32];
     if (threadIdx.x < 32) expT[threadIdx.x] = kExpT[threadIdx.x];
@@ -4416,9 +4432,24 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_exp(StreamArgs a) {
     const int wb = q * run, we = min(wb + run, nW);
     const float* fv = a.fullv + (size_t)r * a.full_stride;
     float* pv = a.fullp + (size_t)r * a.full_stride;
+    const int V = a.vocab;
+    const char* rowp = static_cast<const char*>(a.logits) + (size_t)r * (size_t)a.logits_stride * (DT == 0 ? 4 : 2);
+    const uint32_t* mrow = LAZY && (P.flags & RF_MASK) ? a.mask + (int64_t)r * a.mask_stride : nullptr;
+    // (clamped to the row's last eight ids: a step past them is taken again below)
+    auto fetch = [&](int i0, float (&x)[8], uint32_t& mw) {
+        if (LAZY) {
+            load8<DT>(rowp, min(i0, (V - 8) & ~7), x);
+            mw = mrow != nullptr ? mrow[min(i0, V - 1) >> 5] : 0xFFFFFFFFu;
+        } else {
+            const float4 c0 = reinterpret_cast<const float4*>(fv + i0)[0], c1 = reinterpret_cast<const float4*>(fv + i0)[1];
+            x[0] = c0.x; x[1] = c0.y; x[2] = c0.z; x[3] = c0.w;
+            x[4] = c1.x; x[5] = c1.y; x[6] = c1.z; x[7] = c1.w;
+        }
+    };
     // the first window's first step in flight while the row's maximum is found
-    float4 c0 = reinterpret_cast<const float4*>(fv + wb * WS + lane * 8)[0];
-    float4 c1 = reinterpret_cast<const float4*>(fv + wb * WS + lane * 8)[1];
+    float cx[8];
+    uint32_t cm = 0u;
+    fetch(wb * WS + lane * 8, cx, cm);
     // the row's maximum over the window maxima and, in the same reads, the
     // approximate sum before the first window from k_fs_max's window sums
     // relative to their own maxima (each lane's windows before wb rescaled to
@@ -4457,9 +4488,24 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_exp(StreamArgs a) {
             // the next step's (or window's) values in flight while these are worked on
             const bool more = g + 1 < G || w + 1 < we;
             const int in = more ? (g + 1 < G ? i0 + kFWin : (w + 1) * WS + lane * 8) : i0;
-            const float4 n0 = reinterpret_cast<const float4*>(fv + in)[0];
-            const float4 n1 = reinterpret_cast<const float4*>(fv + in)[1];
-            const float x[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+            float nx[8], x[8];
+            uint32_t nm = 0u;
+            fetch(in, nx, nm);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = cx[j];
+            if (LAZY) {
+                if (i0 + 8 > V) {   // the row's ragged end, and past it
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = i0 + j < V ? load_logit<DT>(rowp, i0 + j) : -__builtin_inff();
+                }
+                if (mrow != nullptr) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = (cm >> ((i0 + j) & 31)) & 1u ? x[j] : -__builtin_inff();
+                }
+                // (the maximum with -inf makes a NaN -inf, as plain_value does)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = fmaxf(x[j] * P.inv_temp, -__builtin_inff());
+            }
             float v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -4516,8 +4562,9 @@ __global__ __launch_bounds__(64 * kFsWaves) void k_fs_exp(StreamArgs a) {
             const XPair sp = wave_scan_pair_any(lp);
             wp = xcomp(wp, XPair{(uint32_t)__builtin_amdgcn_readlane((int)sp.d0, 63),
                                  (uint32_t)__builtin_amdgcn_readlane((int)sp.d1, 63)});
-            c0 = n0;
-            c1 = n1;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cx[j] = nx[j];
+            cm = nm;
         }
         if (cut) {
             emn = wave_min_u32(emn);
@@ -4565,6 +4612,29 @@ __device__ __forceinline__ void wave_ids_ascending(uint32_t* ids, int n, const f
 // rows without penalties, top-p and min-p (the CLI's identity() + temperature: without
 // those stages' code the kernel keeps its state in registers); the other one
 // for the remaining full rows.
+// The transformed row into fv (-inf past V), for a row whose k_fs_max left it out.
+// (plain values, not the argument block: a reference to it would put a copy on
+// every thread's stack)
+__device__ __noinline__ void fill_full(const char* rowp, int dtype, int V, int Vp, const uint32_t* mrow, float inv_temp,
+                                       float* fv) {
+    for (int b = threadIdx.x; b < Vp; b += 4 * kFT) {
+        float x[4];
+        uint32_t mw[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = min(b + q * kFT, V - 1);
+            x[q] = load_logit_dt(rowp, dtype, i);
+            mw[q] = mrow != nullptr ? mrow[i >> 5] : 0xFFFFFFFFu;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = b + q * kFT;
+            if (i < Vp) fv[i] = i < V ? plain_value(x[q], (mw[q] >> (i & 31)) & 1u, inv_temp) : -__builtin_inff();
+        }
+    }
+    __syncthreads();
+}
+
 template <bool GT, bool PRE, bool PLAIN>
 __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -4662,6 +4732,22 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     using BT = std::integral_constant<bool, true>;
     using BF = std::integral_constant<bool, false>;
     constexpr bool pre = PRE;
+    // a.fs_lazy: the transformed row is not in fv until a stage that reads or
+    // writes the whole of it asks for it; single ids are taken from the logits
+    bool have_fv = !(PRE && !PLAIN && a.fs_lazy);
+    auto need_fv = [&]() {
+        if (PRE && !PLAIN && !have_fv) {
+            fill_full(rowp, a.dtype, V, Vp, (P.flags & RF_MASK) ? a.mask + (int64_t)r * a.mask_stride : nullptr, P.inv_temp, fv);
+            have_fv = true;
+        }
+    };
+    auto xat = [&](int i) -> float {
+        if (PRE && !PLAIN && !have_fv) {
+            const bool ok = !(P.flags & RF_MASK) || ((a.mask[(int64_t)r * a.mask_stride + (i >> 5)] >> (i & 31)) & 1u);
+            return plain_value(load_logit_dt(rowp, a.dtype, i), ok, P.inv_temp);
+        }
+        return fv[i];
+    };
     // the draw's window sums of p from the numerators' double sums (rows with
     // penalties take them value by value, as without RF_FPRE)
     const bool sums = PRE && (P.flags & (RF_REP | RF_DRY | RF_FP | RF_BIAS)) == 0;
@@ -4879,6 +4965,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                     __syncthreads();
                     keep = Keep{inv, cut_key, st.sel_need};
                 } else if (need >= neq) {
+                    need_fv();
                     fpass(pv, Vp, [&](int i, float e) {
                         if (__float_as_uint(e * inv) < cut_key) {
                             fv[i] = -__builtin_inff();
@@ -4886,6 +4973,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                         }
                     });
                 } else {
+                    need_fv();
                     // equal keys at the cut, ranked by id: each window's count
                     // of them, the windows' prefix, then each one's rank
                     uint32_t* wc = f.winEF;
@@ -5035,7 +5123,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                     kq[j] = q < n0 && (!eq || eqr < list_need);
                     eqr += eq;
                     ck += kq[j];
-                    if (kq[j]) mk = fmaxf(mk, fv[li_[j]]);
+                    if (kq[j]) mk = fmaxf(mk, xat((int)li_[j]));
                 }
                 mk = wave_max_f(mk);
                 int kpos = wave_incl_sum_i(ck) - ck;
@@ -5045,7 +5133,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                     if (kq[j]) {
                         uint32_t e = le_[j];
                         // numerators relative to m' when the cut left the maximum out
-                        if (mk != m) e = __float_as_uint(libm_expf_t(fv[li_[j]] - mk, st.expT));
+                        if (mk != m) e = __float_as_uint(libm_expf_t(xat((int)li_[j]) - mk, st.expT));
                         ids[kpos] = li_[j];
                         eb[kpos] = e;
                         ++kpos;
@@ -5168,6 +5256,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                 mk = -__builtin_inff();
             } else if (!mk_same) {
                 mk = -__builtin_inff();
+                need_fv();
                 fpass(fv, Vp, [&](int, float x) { mk = fmaxf(mk, x); });
                 mk = fblock_max(mk, st);
             }
@@ -5241,6 +5330,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                 // ids left in are those with p >= thr > 0 (a removed id's p is 0)
                 const float thr = P.min_p * inv;
                 int left = 0;
+                need_fv();
                 const Keep k0 = keep;   // (ids top-p's predicate left out leave the arrays too)
                 fpass(pv, Vp, [&](int i, float e) {
                     if (!(k0(e, i) * inv >= thr)) {
@@ -5316,6 +5406,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             } else {
                 double ws = 0.0;
                 int c = 0;
+                need_fv();
                 wpass2(pv, fv, nW, G, [&](int w, int g, const float (&e)[8], const float (&x)[8]) {
                     const int i0 = w * WS + g * kFWin + lane * 8;
 #pragma unroll
@@ -5507,6 +5598,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             // kept ids and probabilities in index order
             if (a.kept_idx != nullptr) {
                 int pos = 0;
+                need_fv();
                 wpass2(pv, fv, nW, G, [&](int w, int g, const float (&e)[8], const float (&x)[8]) {
                     if (g == 0) pos = (int)wc[w];
                     int c = 0;
@@ -5539,13 +5631,18 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     if (a.fin_idx != nullptr) {
         float* row = static_cast<float*>(const_cast<void*>(a.logits)) + (int64_t)r * a.logits_stride;
         if (listed) {
-            // the kept ids (the list in f.gath, nkept of them) over -inf
+            // the kept ids (the list in f.gath, nkept <= kFSort of them; their
+            // values taken before the row is written over) over -inf
+            static_assert(kFSort <= kFT, "a kept id per thread");
+            const float v = tid < nkept ? xat((int)f.gath[tid]) : 0.0f;
+            __syncthreads();
             for (int i = tid; i < V; i += kFT) row[i] = -__builtin_inff();
             __syncthreads();
-            for (int q = tid; q < nkept; q += kFT) row[f.gath[q]] = fv[f.gath[q]];
+            if (tid < nkept) row[f.gath[tid]] = v;
         } else if (keep.key != 0u) {
-            for (int i = tid; i < V; i += kFT) row[i] = keep(pv[i], i) > 0.0f ? fv[i] : -__builtin_inff();
+            for (int i = tid; i < V; i += kFT) row[i] = keep(pv[i], i) > 0.0f ? xat(i) : -__builtin_inff();
         } else {
+            need_fv();
             for (int i = tid; i < V; i += kFT) row[i] = fv[i];
         }
     }
@@ -5753,7 +5850,9 @@ hipError_t launch_full_pre(const StreamArgs& a, bool plain, bool tp, bool pen, h
     else hipLaunchKernelGGL((k_fs_max<1, false>), g, b, 0, stream, a);
     const int run = fs_run(a.rows, nW), nq = (nW + run - 1) / run;
     const dim3 ge((unsigned)(((int64_t)a.rows * nq + kFsWaves - 1) / kFsWaves));
-    hipLaunchKernelGGL(k_fs_exp, ge, b, 0, stream, a);
+    if (!a.fs_lazy) hipLaunchKernelGGL((k_fs_exp<false, 0>), ge, b, 0, stream, a);
+    else if (a.dtype == 0) hipLaunchKernelGGL((k_fs_exp<true, 0>), ge, b, 0, stream, a);
+    else hipLaunchKernelGGL((k_fs_exp<true, 1>), ge, b, 0, stream, a);
     if (plain) hipLaunchKernelGGL((k_full<false, true, true>), dim3(a.rows), dim3(kFT), (uint32_t)kFullLdsBytes, stream, a);
     if (tp) hipLaunchKernelGGL((k_full<false, true, false>), dim3(a.rows), dim3(kFT), (uint32_t)kFullLdsBytes, stream, a);
     return hipGetLastError();

@@ -151,6 +151,8 @@ struct StreamArgs {
     float* fullp;               // [rows * full_stride] k_full: softmax numerators
     int32_t full_stride;        // k_full: floats per row of fullv / fullp (whole windows of 512 * full_g)
     int32_t full_g;             // k_full: 512-id steps per index-order window
+    int32_t fs_lazy;            // every RF_FPRE row has a top-p or min-p, no penalties and an aligned row:
+                                // the k_fs_* kernels take its values from the logits, fullv is not written
     float* wb_out;              // k_writeback's output for the batch's one row (NULL: in place)
     uint32_t* fs_tab;           // [rows * FS_TABLES * nW] k_fs_* results for k_full's RF_FPRE rows, then
                                 // (16-byte aligned) [rows * nW * 64] uint4 lane tables
