@@ -124,3 +124,30 @@ def test_noalloc_graph_keeps_its_knobs_after_other_calls(hs, wl):
         del g2
     finally:
         s.close()
+
+
+def test_noalloc_penalised_rows_where_the_window_tables_do_not_fit(hs, wl):
+    """Whole-vocabulary rows with penalties beside a top-k row, from batches
+    whose window tables fit the array to the largest it takes without them:
+    that one's rows go through the one-block passes."""
+    V, L = 151936, 16
+    s = hs.Sampler(0, max_rows=64, max_vocab=V)
+    pen = wl.identity_params(temperature=0.8, top_p=0.9, rep_penalty=1.2, repeat_last_n=L)
+    logits = wl._rows_normal(3, 48, V, 3.0)
+    refused = None
+    try:
+        for rows in range(34, 48):
+            plist = [pen] * (rows - 1) + [wl.identity_params(temperature=0.8, top_k=40, rep_penalty=1.2, repeat_last_n=L)]
+            hist = (wl.splitmix64(7, rows * L) % np.uint64(V)).astype(np.int32).reshape(rows, L)
+            w = wl.Workload("noalloc", "f32", logits[:rows], plist, wl.uniform53(9, rows), hist,
+                            np.full(rows, L, np.int64), None)
+            try:
+                ref, got = _both(hs, s, w)
+            except hs.HsampError as e:
+                assert e.status == hs.ERR_CAPACITY
+                refused = rows
+                break
+            _same(ref, got, rows)
+        assert refused is not None and refused > 36
+    finally:
+        s.close()
