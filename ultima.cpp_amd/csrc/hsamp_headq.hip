@@ -29,6 +29,7 @@
 #include <utility>
 
 #include "hsamp_head.h"
+#include "hsamp_wave.h"
 #include "ultima_hsamp.h"
 
 #pragma clang fp contract(off)
@@ -381,8 +382,10 @@ constexpr int shift_class(int j) { return F::BB * j & 3; }
 __device__ __forceinline__ float xadd(float v, int m) { return v + __shfl_xor(v, m, 64); }
 
 // NB: batch rows. Four waves, each with its own 64 / LPR vocabulary rows and
-// its own tile (no barrier: a wave's LDS accesses are in order); the
-// activation's chunk is shared, double-buffered, one barrier per chunk.
+// its own tile (no block barrier: a wave's LDS accesses are in order, and
+// wave_sync keeps the compiler from moving a chunk's stores over the other
+// lanes' reads of the chunk before); the activation's chunk is shared,
+// double-buffered, one barrier per chunk.
 // Lane LPR r + t: row r's lane t.
 //
 // Bound by the vector units (4 to 6 instructions a value: unpack, convert,
@@ -461,6 +464,7 @@ __global__ __launch_bounds__(256) void k_head_q(const unsigned char* __restrict_
         for (int i = 0; i < NS; ++i) a[b][i] = 0.0f;
     uint32_t* mine = tiles[wave];
     for (int c = 0; c < nC; ++c) {
+        wave_sync();                                       // the lanes' reads of the chunk before are done
         tile.store(mine, lane);
         store_x(c & 1);
         __syncthreads();
