@@ -356,7 +356,9 @@ typedef struct ultima_hsamp_head {
     const float* hidden;        /* [rows, hidden_stride] final hidden states */
     int64_t hidden_stride;      /* elements between rows, >= hidden_dim */
     int32_t rows;               /* >= 1 */
-    int32_t hidden_dim;         /* H >= 1 */
+    int32_t hidden_dim;         /* H >= 1; quantised heads: H < 2^30, and the bytes of min(vocab, 32) weight
+                                   rows (16 of the four-lane types: all but Q8_0 and PQ2_0) below 2^32 - 30,
+                                   else ULTIMA_HSAMP_ERR_UNSUPPORTED; PQ2_0: H <= 65536 */
     int32_t vocab;              /* V >= 1 */
     int32_t weight_dtype;       /* ULTIMA_HSAMP_F32, ULTIMA_HSAMP_BF16 or ULTIMA_HSAMP_HEAD_* */
     const float* norm_scale;    /* [H] output-norm weights */

@@ -222,3 +222,19 @@ def test_verify_block_rejects_bad_arguments(pkg):
                 dict(out_tokens=None), dict(out_count=None), dict(draft=None), dict(hist=None),
                 dict(params=ctypes.POINTER(hs.Params)())):
         assert L.ultima_hsamp_verify_block(h, ctypes.byref(mk(**bad)), None) == hs.ERR_INVALID, bad
+
+
+def test_lm_head_refuses_rows_past_32_bit_offsets(pkg):
+    """Quantised heads whose one activation row (H >= 2^30) or whose tile of
+    weight rows (32 of Q8_0, 16 of the K types; as many as the head has) passes
+    the kernels' 32-bit offsets: refused before any device work."""
+    hs = pkg.hsamp
+    p = 16   # never dereferenced
+    h = hs.Head()
+    h.hidden = h.norm_scale = h.weight = h.normed = h.logits = p
+    h.eps, h.logit_scale = 1e-6, 1.0
+    for dt, rows, H, V in [(hs.HEAD_Q4_K, 1, 1 << 30, 1), (hs.HEAD_Q4_K, 5, 1 << 30, 4), (hs.HEAD_Q6_K, 16, 1 << 29, 16),
+                           (hs.HEAD_Q8_0, 1, 1 << 27, 64), (hs.HEAD_Q8_0, 5, 1 << 27, 31), (hs.HEAD_Q5_0, 1, 1 << 29, 16)]:
+        h.weight_dtype, h.rows, h.hidden_dim, h.vocab = dt, rows, H, V
+        h.hidden_stride, h.logits_stride = H, V
+        assert hs.lib().ultima_hsamp_lm_head(ctypes.byref(h), None) == hs.ERR_UNSUPPORTED, (dt, rows, H, V)

@@ -196,6 +196,24 @@ def test_quant_head_many_rows_matches_oracle_bits(hs, name, rows, H, V, offset, 
     np.testing.assert_array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
 
 
+@pytest.mark.parametrize("name,rows,V", [("q4k", 16, 8), ("q8_0", 7, 3)])
+def test_quant_head_rows_past_32_bit_offsets(hs, name, rows, V):
+    """H = 2^26: sixteen activation rows are 2^32 bytes. The first and the last
+    row against the oracle."""
+    import torch
+    H, dt = 1 << 26, O.HEAD_NAMES[name]
+    dev = torch.device("cuda:0")
+    w = np.tile(WL.quant_head(dt, V, 1 << 14, seed=dt), (1, H >> 14))
+    x = torch.empty((rows, H), device=dev)
+    x.normal_(0.0, 2.0, generator=torch.Generator(device=dev).manual_seed(5))
+    g = torch.ones(H, device=dev)
+    got, _ = hs.lm_head(x, g, 1e-6, torch.from_numpy(w).to(dev), weight_dtype=dt)
+    got = got.cpu().numpy()
+    for r in (0, rows - 1):
+        want, _ = O.lm_head(x[r].cpu().numpy(), np.ones(H, np.float32), 1e-6, w, dtype=dt)
+        np.testing.assert_array_equal(got[r].view(np.uint32), want[0].view(np.uint32))
+
+
 @pytest.mark.parametrize("name", ["q8_0", "q4_1", "q5_0", "pq2_0"])
 @pytest.mark.parametrize("H", [96, 1056, 384])
 def test_quant_head_partial_chunks(hs, name, H):

@@ -32,6 +32,8 @@ constexpr int kGemvRows = 4;
 // values / bytes of one block of a quantised head type (0 for others)
 int head_block_values(int dtype);
 int head_block_bytes(int dtype);
+// whether a quantised head's rows are within the kernels' 32-bit offsets
+bool head_quant_fits(const ultima_hsamp_head* h);
 // the final rmsnorm (and the fold, when h->fold_block divides H) of every row
 // into h->normed
 hipError_t launch_head_prep(const ultima_hsamp_head* h, hipStream_t s);

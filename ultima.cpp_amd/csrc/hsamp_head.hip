@@ -357,6 +357,7 @@ extern "C" int ultima_hsamp_lm_head(const ultima_hsamp_head* h, void* hip_stream
     if (h->fold_block > ULTIMA_HSAMP_MAX_FOLD_BLOCK) return ULTIMA_HSAMP_ERR_UNSUPPORTED;
     // row offsets must fit the kernels' 32-bit index arithmetic within a row
     if ((int64_t)h->vocab * h->hidden_dim >= (int64_t)1 << 40) return ULTIMA_HSAMP_ERR_UNSUPPORTED;
+    if (!dense && !head_quant_fits(h)) return ULTIMA_HSAMP_ERR_UNSUPPORTED;
     hipStream_t s = static_cast<hipStream_t>(hip_stream);
     // the fold applies when its block divides H (else the reference leaves
     // the rows as they are)

@@ -24,6 +24,7 @@
 //   and shifts over four values at once) and converted by byte.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 #include <utility>
@@ -294,7 +295,7 @@ constexpr int kMaxPqBlocks = 512;   // PQ2_0 block sums kept in LDS: H <= 65536
 // ---- chunks of rows into LDS -------------------------------------------------------
 // R rows' chunks of PC blocks, loaded by NT threads through one buffer
 // resource based at the first row (16-byte aligned down; `delta` bytes before
-// it): 32-bit offsets, loads past the rows' end read 0. The slots are NV
+// it): 32-bit offsets (offsets_fit), loads past the rows' end read 0. The slots are NV
 // 16-byte vectors padded to S dwords (S = 8 mod 32: the rows' 8-byte reads
 // spread over the banks).
 template <class F, int PC, int R, int NT>
@@ -339,7 +340,7 @@ struct Tile {
     __device__ __forceinline__ void load(int c, int nb) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            uint32_t o = ofs[i] + (uint32_t)(c * CB);
+            uint32_t o = ofs[i] + (uint32_t)c * CB;
             if (!G16) {
                 const uint32_t end = o + (uint32_t)(min(PC, nb - c * PC) * F::BB);
                 o = (o & ~15u) + 16u * (uint32_t)seg[i];
@@ -356,19 +357,21 @@ struct Tile {
     // row r's bytes of chunk c
     template <int AL>
     __device__ __forceinline__ RowBytes<AL> row(const uint32_t* tile, int r, int64_t rb, int c) const {
-        const int sh = (int)((delta + (uint32_t)((int64_t)r * rb) + (uint32_t)(c * CB)) & 15u);
+        const int sh = (int)((delta + (uint32_t)((int64_t)r * rb) + (uint32_t)c * CB) & 15u);
         return {tile + r * S + (sh >> 2), sh & 3};
     }
 };
 
 // n rows of H activation values (H a multiple of 4: a 16-byte load lies inside
 // the rows or past them): loads past the last row read 0, those past a row's
-// end the next row's, which no block uses.
+// end the next row's, which no block uses. 32-bit offsets: n * H * 4 < 2^32
+// (offsets_fit).
 struct Rows {
     __amdgpu_buffer_rsrc_t rs;
     uint32_t row;   // bytes
     __device__ __forceinline__ Rows(const float* x, int n, int H)
-        : rs(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), (short)0, n * H * 4, 0x00020000)),
+        : rs(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), (short)0, (int)((uint32_t)n * (uint32_t)H * 4u),
+                                               0x00020000)),
           row((uint32_t)H * 4u) {}
     __device__ __forceinline__ uint32_t offset(int j, int k) const { return (uint32_t)j * row + 4u * (uint32_t)k; }
     __device__ __forceinline__ u32x4 load(uint32_t o) const { return __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0); }
@@ -428,7 +431,7 @@ __global__ __launch_bounds__(256) void k_head_q(const unsigned char* __restrict_
     }
     auto load_x = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < NX; ++i) xv[i] = xr.load(xo[i] + (uint32_t)(c * CE * 4));
+        for (int i = 0; i < NX; ++i) xv[i] = xr.load(xo[i] + (uint32_t)c * (CE * 4));
     };
     auto store_x = [&](int buf) {
 #pragma unroll
@@ -645,7 +648,7 @@ __global__ __launch_bounds__(256, 2) void k_head_qm(const unsigned char* __restr
     }
     auto load_x = [&](int c) {
 #pragma unroll
-        for (int k = 0; k < NX; ++k) xv[k] = xr.load(xo[k] + (uint32_t)(c * CE * 4));
+        for (int k = 0; k < NX; ++k) xv[k] = xr.load(xo[k] + (uint32_t)c * (CE * 4));
     };
     auto store_x = [&]() {
 #pragma unroll
@@ -790,20 +793,32 @@ hipError_t launch_qm(const ultima_hsamp_head* h, const float* xin, int64_t rb, b
     return hipGetLastError();
 }
 
+// Whether the kernels' 32-bit offsets reach every byte of a tile: its `rows`
+// weight rows of rb bytes (of the V there are; 15 bytes of alignment on either
+// side) and nx activation rows.
+bool offsets_fit(int64_t rb, int rows, int V, int64_t H, int nx) {
+    const int64_t lim = (int64_t)1 << 32;
+    return std::min(rows, V) * rb + 30 < lim && nx * H * 4 < lim;
+}
+
 // Up to kGemvRows rows (PQ2_0, whose block sums are per batch row: any number,
 // four at a time) the vector units, which unpack each value once for all rows;
 // more the matrix cores, a tile of sixteen rows costing the same for five:
-// Q4_K, 4 rows 162 us by the first, 5 rows 295 us by the second.
+// Q4_K, 4 rows 162 us by the first, 5 rows 295 us by the second. Hidden sizes
+// of 2^26 and more, whose sixteen activation rows pass 32-bit offsets, stay on
+// the vector units with as many batch rows at a time as do not.
 template <int T>
 hipError_t launch_q(const ultima_hsamp_head* h, const float* xin, int64_t rb, bool al, hipStream_t s) {
-    if (h->rows == 1) return launch_q_nb<T, 1>(h, xin, rb, al, s);
-    if (h->rows == 2) return launch_q_nb<T, 2>(h, xin, rb, al, s);
-    if constexpr (T == ULTIMA_HSAMP_HEAD_PQ2_0) {
-        return launch_q_nb<T, 4>(h, xin, rb, al, s);
-    } else {
-        if (h->rows <= kGemvRows) return launch_q_nb<T, 4>(h, xin, rb, al, s);
-        return launch_qm<T>(h, xin, rb, al, s);
+    using F = typename FmtOf<T>::F;
+    const int64_t H = h->hidden_dim;
+    auto fits = [&](int nb) { return offsets_fit(rb, 64 / F::LPR, h->vocab, H, nb); };
+    if constexpr (T != ULTIMA_HSAMP_HEAD_PQ2_0) {
+        constexpr int R = F::NA == 64 ? 32 : 64;           // as launch_qm
+        if (h->rows > kGemvRows && offsets_fit(rb, R, h->vocab, H, 16)) return launch_qm<T>(h, xin, rb, al, s);
     }
+    if (h->rows > 2 && fits(4)) return launch_q_nb<T, 4>(h, xin, rb, al, s);
+    if (h->rows > 1 && fits(2)) return launch_q_nb<T, 2>(h, xin, rb, al, s);
+    return launch_q_nb<T, 1>(h, xin, rb, al, s);
 }
 
 // ---- the norm and the fold -------------------------------------------------------
@@ -989,6 +1004,13 @@ int head_block_bytes(int dtype) {
         case ULTIMA_HSAMP_HEAD_PQ2_0: return 34;
         default: return 0;
     }
+}
+
+bool head_quant_fits(const ultima_hsamp_head* h) {
+    const int64_t be = head_block_values(h->weight_dtype), H = h->hidden_dim;
+    const bool two = h->weight_dtype == ULTIMA_HSAMP_HEAD_Q8_0 || h->weight_dtype == ULTIMA_HSAMP_HEAD_PQ2_0;
+    const int lpr = two ? FQ8_0::LPR : FQ4_K::LPR;
+    return H % be != 0 || offsets_fit(H / be * head_block_bytes(h->weight_dtype), 64 / lpr, h->vocab, H, 1);
 }
 
 hipError_t launch_head_prep(const ultima_hsamp_head* h, hipStream_t s) {
