@@ -123,6 +123,19 @@ def test_top_p_rows_read_from_the_logits(sampler, wl, V, dtype, align):
         assert compare_rows(w, g, writeback=wb) == rows
 
 
+@pytest.mark.parametrize("rows,dtype", [(252, "f32"), (253, "f32"), (253, "bf16")])
+def test_whole_row_passes_on_either_side_of_16384_windows(sampler, wl, rows, dtype):
+    """65 windows a row: up to 252 rows the first pass takes the batch's windows
+    in turn, from 253 rows on each row's in blocks of its own (the last block
+    one window)."""
+    V = 33000
+    knobs = [dict(), dict(top_p=0.9), dict(min_p=0.02)]
+    plist = [wl.identity_params(temperature=0.9, **knobs[r % 3]) for r in range(rows)]
+    w = _wl(wl, V, rows, plist, seed=rows, dtype=dtype)
+    g = run_gpu(sampler, w, set_cap=V)
+    assert compare_rows(w, g, rows=[0, 1, 2, 62, 63, 64, 130, rows - 3, rows - 2, rows - 1]) == 10
+
+
 def test_full_vocab_mixed_with_topk_and_greedy_rows(sampler, wl):
     V, rows = 12000, 6
     plist = [wl.identity_params(temperature=1.0, top_p=0.9),

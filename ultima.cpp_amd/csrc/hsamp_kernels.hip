@@ -4287,18 +4287,34 @@ __device__ __forceinline__ float plain_value(float x, bool allowed, float inv_te
 // by each of the row's blocks (L2) and its barriers, 11 us for 16 rows of
 // V = 151936 with 600 ids; the step 205 us against 654 for one block per row
 // that probed a hash table per logit.
-template <int DT, bool PEN>
+// ROW: a row's windows in blocks of its own, the row the block's (always with
+// PEN); else the batch's windows in turn, the row each wave's. With the row the
+// block's, its addresses are scalar, but its plan and arguments come through
+// scalar loads that are waited for before the logits' loads go out: better from
+// 16384 windows on (as fs_run), where the memory's rate counts. V = 151936, us
+// by wave / by block: 16 plain rows 6.2 / 8.4, 32 10.9 / 11.8, 64 16.8 / 15.4,
+// 256 top-p rows 40.7 / 37.8.
+template <int DT, bool PEN, bool ROW>
 __global__ __launch_bounds__(64 * kFsWaves) void k_fs_max(StreamArgs a) {
     __shared__ __attribute__((aligned(16))) uint32_t phit[PEN ? kFsWaves * kFWin : 4];   // table fields, 0: not hit
     __shared__ __attribute__((aligned(16))) float pval[PEN ? kFsWaves * kFWin : 4];      // the hit ids' values
     const int nW = fs_windows(a);
-    const int nb = (nW + kFsWaves - 1) / kFsWaves;         // blocks per row
-    const int r = (int)blockIdx.x / nb, w0 = ((int)blockIdx.x - r * nb) * kFsWaves;
-    const int w = w0 + wave_id();
+    int r, w, w0 = 0;
+    if (ROW) {
+        const int nb = (nW + kFsWaves - 1) / kFsWaves;     // blocks per row
+        r = (int)blockIdx.x / nb;
+        w0 = ((int)blockIdx.x - r * nb) * kFsWaves;
+        w = w0 + wave_id();
+    } else {
+        const int gw = (int)blockIdx.x * kFsWaves + wave_id();
+        r = gw / nW;
+        w = gw - r * nW;
+        if (r >= a.rows) return;
+    }
     const RowPlan P = plan_of(a, r);
     if (!(P.flags & RF_FPRE)) return;
     const bool pen = PEN && (P.flags & (RF_REP | RF_DRY | RF_FP | RF_BIAS)) != 0;
-    if (!pen && w >= nW) return;                           // (a block with penalties keeps all its waves)
+    if (ROW && !pen && w >= nW) return;                    // (a block with penalties keeps all its waves)
     const int lane = lane_id(), V = a.vocab, G = a.full_g, WS = kFWin * G;
     float* fv = a.fullv + (size_t)r * a.full_stride;
     const char* rowp = static_cast<const char*>(a.logits) + (size_t)r * (size_t)a.logits_stride * (DT == 0 ? 4 : 2);
@@ -5843,12 +5859,20 @@ hipError_t launch_merge(const StreamArgs& a, hipStream_t stream) {
 // pen: some of them have penalties or a logit bias.
 hipError_t launch_full_pre(const StreamArgs& a, bool plain, bool tp, bool pen, hipStream_t stream) {
     const int nW = a.full_stride / (kFWin * a.full_g);
-    const dim3 g((unsigned)((int64_t)a.rows * ((nW + kFsWaves - 1) / kFsWaves))), b(64 * kFsWaves);
-    if (a.dtype == 0 && pen) hipLaunchKernelGGL((k_fs_max<0, true>), g, b, 0, stream, a);
-    else if (a.dtype == 0) hipLaunchKernelGGL((k_fs_max<0, false>), g, b, 0, stream, a);
-    else if (pen) hipLaunchKernelGGL((k_fs_max<1, true>), g, b, 0, stream, a);
-    else hipLaunchKernelGGL((k_fs_max<1, false>), g, b, 0, stream, a);
     const int run = fs_run(a.rows, nW), nq = (nW + run - 1) / run;
+    const bool by_row = pen || run > 1;
+    const int64_t blocks = by_row ? (int64_t)a.rows * ((nW + kFsWaves - 1) / kFsWaves)
+                                  : ((int64_t)a.rows * nW + kFsWaves - 1) / kFsWaves;
+    const dim3 g((unsigned)blocks), b(64 * kFsWaves);
+    if (a.dtype == 0) {
+        if (pen) hipLaunchKernelGGL((k_fs_max<0, true, true>), g, b, 0, stream, a);
+        else if (by_row) hipLaunchKernelGGL((k_fs_max<0, false, true>), g, b, 0, stream, a);
+        else hipLaunchKernelGGL((k_fs_max<0, false, false>), g, b, 0, stream, a);
+    } else {
+        if (pen) hipLaunchKernelGGL((k_fs_max<1, true, true>), g, b, 0, stream, a);
+        else if (by_row) hipLaunchKernelGGL((k_fs_max<1, false, true>), g, b, 0, stream, a);
+        else hipLaunchKernelGGL((k_fs_max<1, false, false>), g, b, 0, stream, a);
+    }
     const dim3 ge((unsigned)(((int64_t)a.rows * nq + kFsWaves - 1) / kFsWaves));
     if (!a.fs_lazy) hipLaunchKernelGGL((k_fs_exp<false, 0>), ge, b, 0, stream, a);
     else if (a.dtype == 0) hipLaunchKernelGGL((k_fs_exp<true, 0>), ge, b, 0, stream, a);
