@@ -267,6 +267,105 @@ def test_min_p_at_a_numerators_edge(sampler, wl, sigma, top_p, temp):
         assert compare_rows(w, g, writeback=pen) == len(edges)
 
 
+@pytest.mark.parametrize("sigma,top_p,temp", [(3.0, 1.0, 0.8), (0.5, 0.9, 1.0), (1.5, 0.999, 1.0)])
+def test_min_p_at_a_numerators_edge_of_aligned_rows(sampler, wl, sigma, top_p, temp):
+    """min_p at one id's exp(x - max) and a float to either side, in aligned
+    rows (no transformed copy): with no top-p the threshold times fl(1/S)
+    decides, after it the numerators, or the sum of what it left."""
+    V = 20012
+    row = wl._rows_normal(int(sigma * 10), 1, V, sigma)[0]
+    x = row * np.float32(1.0 / np.float32(temp))
+    e = np.sort(np.exp((x - x.max()).astype(np.float32).astype(np.float64)).astype(np.float32))[::-1]
+    edges = [np.float32(v) for k in (3, 700, 4000) for v in (e[k], np.nextafter(e[k], np.float32(2)), np.nextafter(e[k], np.float32(0)))]
+    edges += [np.float32(v) for v in (1.0, 1.0000001, 2.0, 1e-25, 1e-45, 0.05)]
+    plist = [wl.identity_params(temperature=temp, top_p=top_p, min_p=float(v)) for v in edges]
+    w = _wl(wl, V, len(edges), plist, seed=3)
+    w.logits[:] = row
+    for wb in (False, True):
+        g = run_gpu(sampler, w, writeback=wb, set_cap=V)
+        assert compare_rows(w, g, writeback=wb) == len(edges)
+
+
+def _as(wl, w, dtype):
+    if dtype == "bf16":
+        w.logits, w.dtype = wl.to_bf16_bits(w.logits), dtype
+    return w
+
+
+def _without_sets(sampler, w, g, align=None):
+    """Token, row flags and kept count of the run that asks for no sets."""
+    import torch
+    from gpu_helpers import to_device
+    x, u, h, m = to_device(w)
+    if align:
+        xp = torch.zeros((w.rows, (w.vocab + align - 1) // align * align), dtype=x.dtype, device=x.device)
+        xp[:, :w.vocab] = x
+        x = xp[:, :w.vocab]
+    out = {"kept_count": torch.empty(w.rows, dtype=torch.int32, device=x.device)}
+    o = sampler.run(x, w.params, u, hist=h, hist_len=w.hist_len, mask=m, outputs=out)
+    torch.cuda.synchronize()
+    for k in ("token", "row_flags", "kept_count"):
+        np.testing.assert_array_equal(o[k].cpu().numpy(), g[k], err_msg=k)
+
+
+@pytest.mark.parametrize("V,dtype,align", [(2053, "f32", 4), (30000, "f32", None), (30001, "bf16", 8), (30001, "f32", None)])
+def test_rows_from_which_no_id_leaves(sampler, wl, V, dtype, align):
+    """min-p and top-p that remove nothing, from rows whose numerators are all
+    above 0, underflow to 0 though their logits are finite, or are masked out;
+    kept sets of thousands by top-p and by min-p beside them; the write-back."""
+    # (knobs, sigma of the logits)
+    rows = [(dict(min_p=1e-12), 1.0), (dict(min_p=1e-45), 60.0), (dict(min_p=1e-45, top_p=0.9999999), 60.0),
+            (dict(top_p=0.9999999), 1.0), (dict(top_p=0.9), 0.3), (dict(min_p=0.3), 0.2),
+            (dict(top_p=0.95, min_p=0.3), 0.2), (dict(min_p=1e-12), 1.0)]
+    plist = [wl.identity_params(temperature=0.9, **k) for k, _ in rows]
+    w = _wl(wl, V, len(rows), plist, seed=V, sigma=[s for _, s in rows])
+    w.logits[1:3, 100:103] = 400.0        # fl(1/S) below a half: the threshold rounds to 0
+    w = _as(wl, w, dtype)
+    w.mask = np.full((len(rows), (V + 31) // 32), 0xFFFFFFFF, np.uint32)
+    w.mask[7, ::3] = 0x0FF0F0F1
+    g = run_gpu(sampler, w, set_cap=V, row_align=align)
+    assert compare_rows(w, g) == len(rows)
+    assert int(g["kept_count"][0]) == int(g["kept_count"][1]) == V and int(g["kept_count"][7]) < V
+    assert 512 < min(int(g["kept_count"][r]) for r in (4, 5, 6))
+    _without_sets(sampler, w, g, align)
+    if dtype == "f32":
+        g = run_gpu(sampler, w, writeback=True, set_cap=V, row_align=align)
+        assert compare_rows(w, g, writeback=True) == len(rows)
+
+
+@pytest.mark.parametrize("V,dtype,align", [(30001, "f32", 4), (30001, "bf16", 8), (30001, "f32", None)])
+def test_nan_logits_in_top_p_and_min_p_rows(hs, sampler, wl, V, dtype, align):
+    """NaN logits count as -inf and flag the row, also where the transformed
+    row is not kept: the outputs are those of the row with the NaN ids masked
+    out (checked against the oracle), but for the flag."""
+    knobs = [(dict(top_p=0.9), 2.0), (dict(top_p=0.9), 0.2), (dict(min_p=0.05), 2.0), (dict(min_p=0.3), 0.2),
+             (dict(min_p=1e-12), 1.0), (dict(top_p=0.9, min_p=1e-45), 60.0), (dict(min_p=1e-45), 60.0)]
+    n = len(knobs)
+    w = _wl(wl, V, n, [wl.identity_params(temperature=0.8, **k) for k, _ in knobs], seed=9, sigma=[s for _, s in knobs])
+    w.logits[5:, 100:110] = 400.0
+    w = _as(wl, w, dtype)
+    at = [0, 5, 512, 2047, V - 1] + [int(i) for r in range(n) for i in np.argsort(w.logits_f32()[r])[-3:]]
+    w.mask = np.full((n, (V + 31) // 32), 0xFFFFFFFF, np.uint32)
+    for i in at:
+        w.mask[:, i // 32] &= np.uint32(0xFFFFFFFF) ^ np.uint32(1 << (i % 32))
+    want = run_gpu(sampler, w, set_cap=V, row_align=align)
+    assert compare_rows(w, want) == n
+    w.mask = None
+    x = w.logits_f32().copy()
+    x[:, at] = np.nan
+    w.logits = x if dtype == "f32" else wl.to_bf16_bits(np.where(np.isnan(x), np.float32(0), x))
+    if dtype == "bf16":
+        w.logits[:, at] = 0x7FC0
+    got = run_gpu(sampler, w, set_cap=V, row_align=align)
+    for r in range(n):
+        c = int(want["kept_count"][r])
+        assert int(got["token"][r]) == int(want["token"][r]) and int(got["kept_count"][r]) == c, r
+        np.testing.assert_array_equal(got["kept_idx"][r][:c], want["kept_idx"][r][:c])
+        np.testing.assert_array_equal(got["kept_prob"][r][:c].view(np.uint32), want["kept_prob"][r][:c].view(np.uint32))
+        assert int(got["row_flags"][r]) == int(want["row_flags"][r]) | hs.ROW_NAN, r
+    _without_sets(sampler, w, got, align)
+
+
 def test_full_vocab_draw_without_sets(sampler, wl):
     """With no kept set asked for, rows whose top-p or min-p removed ids take
     the draw's window sums from the numerators alone and their kept count from

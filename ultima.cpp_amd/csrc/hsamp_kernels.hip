@@ -4622,35 +4622,45 @@ __device__ __forceinline__ void wave_ids_ascending(uint32_t* ids, int n, const f
     wave_sync();
 }
 
+// The transformed row into fv (-inf past V), for a row whose k_fs_max left it
+// out (V >= 8, the row 16-byte aligned). (plain values, not the argument block:
+// a reference to it would put a copy on every thread's stack)
+template <int DT>
+__device__ __noinline__ void fill_full(const char* rowp, int V, int Vp, const uint32_t* mrow, float inv_temp, float* fv) {
+    for (int b = 8 * (int)threadIdx.x; b < Vp; b += 16 * kFT) {
+        float x[2][8];
+        uint32_t mw[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int i0 = b + q * 8 * kFT;
+            load8<DT>(rowp, min(i0, (V - 8) & ~7), x[q]);
+            mw[q] = mrow != nullptr ? mrow[min(i0, V - 1) >> 5] : 0xFFFFFFFFu;   // (eight ids share one mask word)
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int i0 = b + q * 8 * kFT;
+            if (i0 >= Vp) break;
+            if (i0 + 8 > V) {   // the row's ragged end, and past it
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[q][j] = i0 + j < V ? load_logit<DT>(rowp, i0 + j) : -__builtin_inff();
+            }
+            float y[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) y[j] = plain_value(x[q][j], (mw[q] >> ((i0 + j) & 31)) & 1u, inv_temp);
+            float4* dst = reinterpret_cast<float4*>(fv + i0);
+            dst[0] = make_float4(y[0], y[1], y[2], y[3]);
+            dst[1] = make_float4(y[4], y[5], y[6], y[7]);
+        }
+    }
+    __syncthreads();
+}
+
 // Full-vocabulary rows, one block of kFT threads per row. PRE: the
 // instantiations for the RF_FPRE rows (k_fs_* did the transform and left the
 // window tables; no top-k), PLAIN among them for the
 // rows without penalties, top-p and min-p (the CLI's identity() + temperature: without
 // those stages' code the kernel keeps its state in registers); the other one
 // for the remaining full rows.
-// The transformed row into fv (-inf past V), for a row whose k_fs_max left it out.
-// (plain values, not the argument block: a reference to it would put a copy on
-// every thread's stack)
-__device__ __noinline__ void fill_full(const char* rowp, int dtype, int V, int Vp, const uint32_t* mrow, float inv_temp,
-                                       float* fv) {
-    for (int b = threadIdx.x; b < Vp; b += 4 * kFT) {
-        float x[4];
-        uint32_t mw[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int i = min(b + q * kFT, V - 1);
-            x[q] = load_logit_dt(rowp, dtype, i);
-            mw[q] = mrow != nullptr ? mrow[i >> 5] : 0xFFFFFFFFu;
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int i = b + q * kFT;
-            if (i < Vp) fv[i] = i < V ? plain_value(x[q], (mw[q] >> (i & 31)) & 1u, inv_temp) : -__builtin_inff();
-        }
-    }
-    __syncthreads();
-}
-
 template <bool GT, bool PRE, bool PLAIN>
 __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -4753,7 +4763,9 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     bool have_fv = !(PRE && !PLAIN && a.fs_lazy);
     auto need_fv = [&]() {
         if (PRE && !PLAIN && !have_fv) {
-            fill_full(rowp, a.dtype, V, Vp, (P.flags & RF_MASK) ? a.mask + (int64_t)r * a.mask_stride : nullptr, P.inv_temp, fv);
+            const uint32_t* mrow = (P.flags & RF_MASK) ? a.mask + (int64_t)r * a.mask_stride : nullptr;
+            if (a.dtype == 0) fill_full<0>(rowp, V, Vp, mrow, P.inv_temp, fv);
+            else fill_full<1>(rowp, V, Vp, mrow, P.inv_temp, fv);
             have_fv = true;
         }
     };
@@ -4768,13 +4780,14 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
     // penalties take them value by value, as without RF_FPRE)
     const bool sums = PRE && (P.flags & (RF_REP | RF_DRY | RF_FP | RF_BIAS)) == 0;
     static_assert(kFMaxWin <= 2 * kFT, "two windows per thread");
-    double sdr[2] = {0.0, 0.0};   // PRE: the draw's window sums of the numerators ...
+    double sdr[2] = {0.0, 0.0};   // PLAIN: the draw's window sums of the numerators ...
     uint32_t cnr[2] = {0u, 0u};   // ... and counts (windows tid, tid + kFT)
     uint32_t emn = 0xFFFFFFFFu;   // PRE: the smallest numerator above 0 of those windows
     if constexpr (PRE) {
         // k_fs_* transformed the row and left its window tables, all loaded at
         // once: maxima and NaN flags for the row's maximum, the exact sum's
-        // binades and pairs into LDS, the draw's sums and counts kept here
+        // binades and pairs into LDS, PLAIN rows' sums and counts for the draw
+        // kept here
         const uint32_t* wm = fs_table(a, r, FS_MAX);
         const uint32_t* wn = fs_table(a, r, FS_NAN);
         const uint32_t* we = fs_table(a, r, FS_EF);
@@ -4788,9 +4801,12 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             const int k = tid + i * kFT;
             if (k < nW) {
                 const uint32_t mx = wm[k], nn = wn[k], ef = we[k], d0 = w0[k], d1 = w1[k];
-                sdr[i] = wsd[k];
-                cnr[i] = wcn[k];
-                if (!PLAIN) emn = min(emn, wen[k]);
+                if (PLAIN) {
+                    sdr[i] = wsd[k];
+                    cnr[i] = wcn[k];
+                } else {
+                    emn = min(emn, wen[k]);
+                }
                 mloc = fmaxf(mloc, __uint_as_float(mx));
                 nanv |= nn != 0u;
                 f.winEF[k] = ef;
@@ -5043,39 +5059,57 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             }
         }
 
-        // ---- min-p (sampler.cpp:167-176) from the numerators, without the sum
-        // S' of what top-p left: an id leaves when fl(e fl(1/S')) <
-        // fl(min_p fl(1/S')) (the largest p is fl(1/S'): its e is 1). For
-        // e >= min_p that is never so (rounding is monotone), for
-        // e < min_p (1 - 2^-21) always (the products differ by more than two
-        // of their ulps); when an e lies between, the stage below takes S'.
-        // One pass and a predicate instead of the sum, a pass of writes and
-        // another sum.
-        bool mp_done = false;
-        if (!PLAIN && mpf && mk_same && list_need < 0) {
-            const float lo = P.min_p * (1.0f - 0x1p-21f);
+        // the ids in before min-p when no stage has counted them: the finite
+        // transformed logits (PRE: k_fs_max's counts, which the refresh has not
+        // written over yet)
+        auto count_in = [&]() -> int {
+            int c = 0;
+            if (PRE) {
+                const uint32_t* wcn = fs_table(a, r, FS_CNT);
+                for (int k = tid; k < nW; k += kFT) c += (int)wcn[k];
+            } else {
+                fpass(fv, Vp, [&](int, float x) { c += x != -__builtin_inff(); });
+            }
+            return fblock_sum_i(c, st);
+        };
+
+        // ---- min-p (sampler.cpp:167-176) by one counting pass and a predicate
+        // (the largest p is fl(1/S'): its e is 1): an id leaves when
+        // fl(e fl(1/S')) < fl(min_p fl(1/S')), S' the sum of what top-p left.
+        // When top-p removed nothing S' is S. Else, without S': for e >= min_p
+        // that is never so (rounding is monotone), for e < min_p (1 - 2^-21)
+        // always (the products differ by more than two of their ulps); when an
+        // e lies between, the stage below takes S'.
+        bool mp_done = false, mp_counted = false;
+        if (!PLAIN && (P.flags & RF_MINP) && list_need < 0 && (touched ? mpf && mk_same : fabsf(m) < __builtin_inff())) {
+            const float inv = 1.0f / S, thr = P.min_p * inv;
             int left = 0, amb = 0;
-            fpass(pv, Vp, [&](int i, float e) {
-                if (e >= P.min_p) left += keep(e, i) > 0.0f;
-                else amb += e >= lo;
-            });
-            left = fblock_sum_i(left, st);
-            amb = fblock_sum_i(amb, st);
-            mp_done = amb == 0;
-            // (top-p's predicate may be the tighter one: then no id leaves)
-            if (mp_done && (keep.key == 0u || P.min_p * keep.inv > __uint_as_float(keep.key))) {
-                if (nleft < 0) {
-                    int c = 0;
-                    if (pre) c = (int)(cnr[0] + cnr[1]);
-                    else fpass(fv, Vp, [&](int, float x) { c += x != -__builtin_inff(); });
-                    nleft = fblock_sum_i(c, st);
+            mp_done = !touched && !(thr > 0.0f);   // (a threshold of 0 removes nothing)
+            if (!mp_done) {
+                if (!touched) {
+                    fpass(pv, Vp, [&](int, float e) { left += e * inv >= thr; });
+                } else {
+                    const float lo = P.min_p * (1.0f - 0x1p-21f);
+                    fpass(pv, Vp, [&](int i, float e) {
+                        if (e >= P.min_p) left += keep(e, i) > 0.0f;
+                        else amb += e >= lo;
+                    });
                 }
+                left = fblock_sum_i(left, st);
+                amb = fblock_sum_i(amb, st);
+                mp_done = amb == 0;
+                mp_counted = mp_done;
+            }
+            // (top-p's predicate may be the tighter one: then no id leaves)
+            if (mp_counted && (keep.key == 0u || P.min_p * keep.inv > __uint_as_float(keep.key))) {
+                if (nleft < 0) nleft = count_in();
                 if (left != nleft) {
-                    keep = Keep{1.0f, __float_as_uint(P.min_p), 0x7FFFFFFF};
+                    keep = touched ? Keep{1.0f, __float_as_uint(P.min_p), 0x7FFFFFFF}
+                                   : Keep{inv, __float_as_uint(thr), 0x7FFFFFFF};
                     nleft = left;
                     changed = true;
                     touched = true;
-                    if (left <= kFSort) list_need = left;   // (list_key 0: every one stays)
+                    if (left > 0 && left <= kFSort) list_need = left;   // (list_key 0: every one stays)
                 }
             }
         }
@@ -5117,8 +5151,8 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                 else if (n0 <= 128) wave_ids_ascending<2>(ids, n0, pv, eb);
                 else if (n0 <= 256) wave_ids_ascending<4>(ids, n0, pv, eb);
                 else wave_ids_ascending<8>(ids, n0, pv, eb);
-                // the candidates with p* past the first `need` of them leave;
-                // the largest kept logit m'; the rest close ranks
+                // the candidates with p* past the first `need` of them leave; the
+                // rest close ranks
                 uint32_t li_[8], le_[8];
                 bool kq[8];
                 int ce = 0;
@@ -5131,7 +5165,6 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                 }
                 int eqr = wave_incl_sum_i(ce) - ce;   // equal keys before this lane's first entry
                 int ck = 0;
-                float mk = -__builtin_inff();
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const int q = lane * 8 + j;
@@ -5139,29 +5172,40 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                     kq[j] = q < n0 && (!eq || eqr < list_need);
                     eqr += eq;
                     ck += kq[j];
-                    if (kq[j]) mk = fmaxf(mk, xat((int)li_[j]));
                 }
-                mk = wave_max_f(mk);
                 int kpos = wave_incl_sum_i(ck) - ck;
                 wave_sync();
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     if (kq[j]) {
-                        uint32_t e = le_[j];
-                        // numerators relative to m' when the cut left the maximum out
-                        if (mk != m) e = __float_as_uint(libm_expf_t(xat((int)li_[j]) - mk, st.expT));
                         ids[kpos] = li_[j];
-                        eb[kpos] = e;
+                        eb[kpos] = le_[j];
                         ++kpos;
                     }
                 }
                 int n = __builtin_amdgcn_readlane(kpos, 63);
                 wave_sync();
-                XState s2{-126, 0u};
-                chain_replay(s2, eb, n, __builtin_inff());
-                float inv2 = 1.0f / xs_value(s2);
-                if (!PLAIN && (P.flags & RF_MINP)) {
-                    // min-p on the list (its largest p is fl(1 * inv2))
+                if (!mk_same) {
+                    // the largest kept logit m'; numerators relative to it when
+                    // the cut left the maximum out
+                    float mk = -__builtin_inff();
+#pragma unroll 1
+                    for (int q = lane; q < n; q += 64) mk = fmaxf(mk, xat((int)ids[q]));
+                    mk = wave_max_f(mk);
+                    if (mk != m) {
+#pragma unroll 1
+                        for (int q = lane; q < n; q += 64) eb[q] = __float_as_uint(libm_expf_t(xat((int)ids[q]) - mk, st.expT));
+                    }
+                    wave_sync();
+                }
+                // the sum, and, when min-p is to come after top-p, min-p on the list
+                // (its largest p is fl(1 * inv2)) and the sum of what it left
+                float inv2;
+                for (bool mp = !PLAIN && (P.flags & RF_MINP) && !mp_done;; mp = false) {
+                    XState s2{-126, 0u};
+                    chain_replay(s2, eb, n, __builtin_inff());
+                    inv2 = 1.0f / xs_value(s2);
+                    if (!mp) break;
                     const float thr = P.min_p * inv2;
                     bool k2[8];
                     int c2 = 0;
@@ -5175,22 +5219,18 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                     }
                     const int i2 = wave_incl_sum_i(c2);
                     const int n2 = __builtin_amdgcn_readlane(i2, 63);
-                    if (n2 != n) {
-                        int at = i2 - c2;
-                        wave_sync();
+                    if (n2 == n) break;
+                    int at = i2 - c2;
+                    wave_sync();
 #pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            if (k2[j]) {
-                                ids[at] = li_[j];
-                                eb[at] = le_[j];
-                                ++at;
-                            }
-                        n = n2;
-                        wave_sync();
-                        s2 = XState{-126, 0u};
-                        chain_replay(s2, eb, n, __builtin_inff());
-                        inv2 = 1.0f / xs_value(s2);
-                    }
+                    for (int j = 0; j < 8; ++j)
+                        if (k2[j]) {
+                            ids[at] = li_[j];
+                            eb[at] = le_[j];
+                            ++at;
+                        }
+                    n = n2;
+                    wave_sync();
                 }
                 // the draw (sampler.cpp:178-182): q = p / S_d over the kept ids in index order
                 float pq[8];
@@ -5332,33 +5372,33 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             const float inv = 1.0f / S;
             // (a threshold of 0 -- min_p * inv below the smallest float -- removes nothing)
             if (m != -__builtin_inff() && P.min_p * inv > 0.0f) {
-                if (nleft < 0) {
-                    // the ids in before min-p: the finite transformed logits
-                    int c = 0;
-                    if (pre) {
-                        c = (int)(cnr[0] + cnr[1]);
-                    } else {
-                        fpass(fv, Vp, [&](int, float x) { c += x != -__builtin_inff(); });
-                    }
-                    nleft = fblock_sum_i(c, st);
-                }
+                if (nleft < 0) nleft = count_in();
                 // the largest p is the largest logit's, fl(1 * inv) = inv; the
                 // ids left in are those with p >= thr > 0 (a removed id's p is 0)
                 const float thr = P.min_p * inv;
-                int left = 0;
-                need_fv();
-                const Keep k0 = keep;   // (ids top-p's predicate left out leave the arrays too)
+                int all = 0, left = 0;
                 fpass(pv, Vp, [&](int i, float e) {
-                    if (!(k0(e, i) * inv >= thr)) {
-                        fv[i] = -__builtin_inff();
-                        pv[i] = 0.0f;
-                    } else {
-                        ++left;
-                    }
+                    const bool p = e * inv >= thr;
+                    all += p;
+                    left += p && keep(e, i) > 0.0f;
                 });
-                keep = kKeepAll;
+                all = fblock_sum_i(all, st);
                 left = fblock_sum_i(left, st);
                 changed = left != nleft;
+                if (changed && all == left && fabsf(m) < __builtin_inff()) {
+                    keep = Keep{inv, __float_as_uint(thr), 0x7FFFFFFF};   // (all of them are in top-p's set)
+                } else if (changed) {
+                    need_fv();
+                    const Keep k0 = keep;   // (ids top-p's predicate left out leave the arrays too)
+                    fpass(pv, Vp, [&](int i, float e) {
+                        if (!(k0(e, i) * inv >= thr)) {
+                            fv[i] = -__builtin_inff();
+                            pv[i] = 0.0f;
+                        }
+                    });
+                    __syncthreads();
+                    keep = kKeepAll;
+                }
                 nleft = left;
                 touched |= changed;
             }
@@ -5375,7 +5415,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             const float inv = 1.0f / S;
             double* wq = reinterpret_cast<double*>(f.winA);   // [kFMaxWin] window sums of p, then prefixes
             uint32_t* wc = f.winEF;                            // [kFMaxWin] kept counts, then prefixes
-            if (PRE && (PLAIN || sums) && !touched && !(P.flags & (RF_TOPP | RF_MINP))) {
+            if (PLAIN) {
                 // k_fs_* left each window's numerators summed in double and
                 // its count: the window sums of p are taken as fl(1/S) times
                 // those (within 2^-24 of the sums of fl(e fl(1/S)) relative,
@@ -5419,10 +5459,24 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                         ws = 0.0;
                     }
                 });
+            } else if (PRE && !touched) {
+                // k_fs_* counted the ids left in; the sums value by value
+                const uint32_t* wcn = fs_table(a, r, FS_CNT);
+                double ws = 0.0;
+                wpass(pv, nW, G, [&](int w, int g, const float (&e)[8]) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) ws += (double)(e[j] * inv);
+                    if (g == G - 1) {
+                        ws = wave_sum_d(ws);
+                        if (lane == 0) wq[w] = ws;
+                        ws = 0.0;
+                    }
+                });
+                for (int k = tid; k < nW; k += kFT) wc[k] = wcn[k];
             } else {
+                // (removed ids without a predicate: the stage that removed them has written fv)
                 double ws = 0.0;
                 int c = 0;
-                need_fv();
                 wpass2(pv, fv, nW, G, [&](int w, int g, const float (&e)[8], const float (&x)[8]) {
                     const int i0 = w * WS + g * kFWin + lane * 8;
 #pragma unroll
@@ -5614,18 +5668,17 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
             // kept ids and probabilities in index order
             if (a.kept_idx != nullptr) {
                 int pos = 0;
-                need_fv();
-                wpass2(pv, fv, nW, G, [&](int w, int g, const float (&e)[8], const float (&x)[8]) {
+                auto put = [&](int w, int g, const float (&e)[8], auto in) {
                     if (g == 0) pos = (int)wc[w];
                     int c = 0;
                     const int i0 = w * WS + g * kFWin + lane * 8;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) c += inset(e[j], x[j], i0 + j);
+                    for (int j = 0; j < 8; ++j) c += in(j, i0 + j);
                     const int li = wave_incl_sum_i(c);
                     int p = pos + li - c;
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
-                        if (inset(e[j], x[j], i0 + j)) {
+                        if (in(j, i0 + j)) {
                             if (p < a.set_cap) {
                                 a.kept_idx[(int64_t)r * a.set_cap + p] = i0 + j;
                                 a.kept_prob[(int64_t)r * a.set_cap + p] = e[j] * inv;
@@ -5634,7 +5687,20 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
                         }
                     }
                     pos += __builtin_amdgcn_readlane(li, 63);
-                });
+                };
+                // the numerators alone tell the ids left in: by the predicate, or
+                // where no id left though min-p's threshold was above 0
+                const bool by_e = PRE && !PLAIN && (keep.key != 0u || (!touched && mp_counted));
+                if (by_e) {
+                    wpass(pv, nW, G, [&](int w, int g, const float (&e)[8]) {
+                        put(w, g, e, [&](int j, int i) { return keep(e[j], i) > 0.0f; });
+                    });
+                } else {
+                    need_fv();
+                    wpass2(pv, fv, nW, G, [&](int w, int g, const float (&e)[8], const float (&x)[8]) {
+                        put(w, g, e, [&](int j, int i) { return inset(e[j], x[j], i); });
+                    });
+                }
             }
         }
     }
@@ -5658,8 +5724,7 @@ __global__ __launch_bounds__(kFT) void k_full(StreamArgs a) {
         } else if (keep.key != 0u) {
             for (int i = tid; i < V; i += kFT) row[i] = keep(pv[i], i) > 0.0f ? xat(i) : -__builtin_inff();
         } else {
-            need_fv();
-            for (int i = tid; i < V; i += kFT) row[i] = fv[i];
+            for (int i = tid; i < V; i += kFT) row[i] = xat(i);
         }
     }
     if (wid == 0) emit_token_wave(a, r, tok);
