@@ -399,6 +399,46 @@ def test_reference_cases_through_sample_host(sampler, case):
     np.testing.assert_array_equal(after.view(np.uint32), tr.logits_after.view(np.uint32))
 
 
+def _host_call(s, V, p, hist, bias=None, u=0.37, seed=1, writeback=True):
+    x = np.random.default_rng(seed).normal(0, 2.5, V).astype(np.float32)
+    tr = O.sample_row(x, p, hist=hist, bias=bias, u=u)
+    tok, after = s.sample_host(x, p, hist=hist, bias=bias, u=u, writeback=writeback)
+    assert tok == tr.token or tr.cdf_margin <= 1e-6
+    np.testing.assert_array_equal(after.view(np.uint32), (tr.logits_after if writeback else x).view(np.uint32))
+
+
+@pytest.mark.parametrize("V", [1, 2047, 2049, 6145, 151935])
+@pytest.mark.parametrize("kind", ["server", "open", "greedy", "greedy_plain", "plain_topk"])
+def test_sample_host_writes_back_the_reference_state(sampler, V, kind):
+    """Host rows over several blocks of the write-back and ragged ends: the
+    token and every logit as sample() leaves them, stored straight to host
+    memory or, for whole-vocabulary rows, copied there by a kernel."""
+    p = {"server": O.default_params(temperature=0.8),
+         "open": O.identity_params(temperature=0.8, top_p=0.95, min_p=0.01, rep_penalty=1.2, repeat_last_n=600),
+         "greedy": O.default_params(temperature=0.0, frequency_penalty=0.3),
+         "greedy_plain": O.identity_params(temperature=0.0),
+         "plain_topk": O.identity_params(temperature=1.1, top_k=50)}[kind]
+    rng = np.random.default_rng(V)
+    hist = rng.integers(-2, V + 2, 600).astype(np.int32)
+    hist[-6:] = [0, V - 1, V, -1, min(2048, V - 1), min(2047, V - 1)]
+    bias = {0: 1.5, V - 1: -np.inf} if kind in ("server", "greedy") and V > 1 else None
+    for wb in (True, False):
+        _host_call(sampler, V, p, hist, bias, seed=V, writeback=wb)
+
+
+def test_sample_host_with_a_history_past_its_area(hs):
+    """A session whose history outgrows the staging area made with the handle
+    (1024 ids beside the row), then shorter calls and another vocabulary."""
+    V = 5003
+    s = hs.Sampler(0, max_rows=1, max_vocab=V)
+    hist = np.random.default_rng(4).integers(0, V, 9000).astype(np.int32)
+    p = O.default_params(temperature=0.9, dry_last_n=2048, repeat_last_n=256)
+    for n in (0, 1000, 1024, 1025, 1040, 1056, 1200, 2100, 9000, 40, 0):
+        _host_call(s, V, p, hist[:n], seed=n)
+    _host_call(s, 1001, p, hist[:3000] % 1001, seed=3)
+    s.close()
+
+
 def test_default_params_sample_host(sampler):
     l = np.array([0.1, 0.5, 0.9, 0.3, 0.7, 0.2, 0.4, 0.6, 0.8, 0.15], np.float32)
     for seed in range(20):

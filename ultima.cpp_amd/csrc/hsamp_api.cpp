@@ -737,8 +737,11 @@ int grow(ultima_hsamp* h, bool capturing, T*& ptr, size_t& have, size_t need) {
 // sample_host's staging of V logits and L history ids, and the offset of the history
 size_t stage_hist(int32_t V) { return 64 + (((size_t)V * 4 + 63) & ~size_t(63)); }
 size_t stage_bytes(int32_t V, size_t L) { return (stage_hist(V) + L * 4 + 63) & ~size_t(63); }
-int grow_stage(ultima_hsamp* h, size_t n) {
-    if (n <= h->stage_cap) return ULTIMA_HSAMP_OK;
+// (room for twice the history, so that a growing one moves the area seldom and
+// not every 16 ids)
+int grow_stage(ultima_hsamp* h, int32_t V, size_t L) {
+    if (stage_bytes(V, L) <= h->stage_cap) return ULTIMA_HSAMP_OK;
+    const size_t n = stage_bytes(V, 2 * L);
     if (h->d_stage) HIP_TRY(hipFree(h->d_stage));
     if (h->h_stage) HIP_TRY(hipHostFree(h->h_stage));
     h->d_stage = nullptr;
@@ -863,7 +866,7 @@ int ultima_hsamp_create(int device, int32_t max_rows, int32_t max_vocab, ultima_
     CREATE_TRY(hipMalloc(reinterpret_cast<void**>(&h->fin_idx), (size_t)max_rows * kLimitK * 4));
     CREATE_TRY(hipMalloc(reinterpret_cast<void**>(&h->fin_n), (size_t)max_rows * 4));
     CREATE_TRY(hipHostMalloc(reinterpret_cast<void**>(&h->h_tok), 64, hipHostMallocDefault));
-    if (grow_stage(h, stage_bytes(max_vocab, 1024)) != ULTIMA_HSAMP_OK) return fail(ULTIMA_HSAMP_ERR_NOMEM);
+    if (grow_stage(h, max_vocab, 512) != ULTIMA_HSAMP_OK) return fail(ULTIMA_HSAMP_ERR_NOMEM);
     CREATE_TRY(hipDeviceSynchronize());
 #undef CREATE_TRY
     *out = h;
@@ -1035,7 +1038,7 @@ int ultima_hsamp_sample_host(ultima_hsamp* h, float* logits, int32_t vocab,
     // of them were half of a 156 us call at V = 151936, 92 us now.)
     hipStream_t s = h->own_stream;
     const size_t L = (size_t)params->hist_len, n = stage_bytes(vocab, L);
-    int st = grow_stage(h, n);
+    int st = grow_stage(h, vocab, L);
     if (st != ULTIMA_HSAMP_OK) return st;
     float* h_row = reinterpret_cast<float*>(h->h_stage + 64);
     std::memcpy(h->h_stage, &u, 8);
