@@ -259,6 +259,46 @@ def test_u_on_and_beside_cdf_boundaries(sampler, wl, k, kernel_mode):
     assert compare_rows(w, g, strict_token=True) == B
 
 
+@pytest.mark.parametrize("k,temp", [(300, 0.9), (300, 3.0), (1000, 1.0), (1024, 4.0)])
+def test_draw_near_a_boundary_is_decided_by_the_tree_sums(sampler, wl, k, temp):
+    """The block finalize takes the sequential sums only within 1e-11 of a
+    partial sum (or of the flag's 1e-6 from one); beside that its tree sums
+    decide the token and CDF_NEAR. u at 2e-11 .. 1.9e-6 to either side of
+    partial sums, at 1e-6 +- 1e-10 .. 1e-12 from them (the flag's own edge, on
+    both sides of the margin), near 0 and near 1: every token and every
+    CDF_NEAR flag is the oracle's."""
+    V = 151936
+    base = np.random.default_rng(k).normal(0, 1.5, size=(1, V)).astype(np.float32)
+    base[0, V - 1] = 1e-3 + base[0].max()         # (the last id is kept: its partial sum is 1)
+    params = wl.identity_params(top_k=k, temperature=temp)
+    tr = O.sample_row(base[0], params, u=0.5)
+    p = tr.kept_prob.astype(np.float64)
+    assert p.size == k and int(tr.kept_idx[-1]) == V - 1
+    S = 0.0
+    for v in p:
+        S += v
+    cp, acc = [], 0.0
+    for v in p:
+        acc += v / S
+        cp.append(acc)
+    edge = [1e-6 + d for d in (1e-10, 2e-11, 5e-12, 1e-12, -1e-12, -5e-12, -2e-11, -1e-10)]
+    us = []
+    for j in (0, 1, 17, k // 3, k // 2, k - 3, k - 2):
+        for d in [2e-11, 1e-10, 1e-9, 5e-7, 9.9e-7, 1.01e-6, 1.9e-6] + edge:
+            us += [cp[j] + d, cp[j] - d]
+    us += edge + [1.0 - d for d in edge] + [2e-11, 1.0 - 2e-11, 1.0 - 2.0**-53]
+    us = [u for u in us if 0.0 < u < 1.0]
+    B = len(us)
+    w = _wl_from(wl, np.repeat(base, B, axis=0), [params] * B, us)
+    g = run_gpu(sampler, w)
+    assert compare_rows(w, g, rows=range(0, B, 40), strict_token=True)
+    for r, u in enumerate(us):
+        t = O.sample_row(base[0], params, u=float(u))
+        assert int(g["token"][r]) == t.token, (r, u)
+        # (the oracle's margin: the distance to the nearer of the partial sums around u)
+        assert bool(int(g["row_flags"][r]) & 4) == (t.cdf_margin <= 1e-6), (r, u, t.cdf_margin)
+
+
 @pytest.mark.parametrize("k,top_p,min_p,sigma", [(1000, 0.5, 0.0, 0.01), (900, 0.97, 0.0, 0.3),
                                                  (700, 1.0, 0.9, 0.02), (1024, 0.8, 0.5, 0.05)])
 def test_general_finalize_long_sums(sampler, wl, k, top_p, min_p, sigma):
