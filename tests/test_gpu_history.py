@@ -223,3 +223,67 @@ def test_graph_from_the_first_token(hs, sampler, kernel_mode):
         n = int(got_len[r])
         assert n == P0 + 601
         np.testing.assert_array_equal(got[r, :n], host[r][-n:])
+
+
+@pytest.mark.parametrize("mode", ["run", "commit", "captured"])
+def test_whole_vocabulary_rows_with_device_history(hs, sampler, mode):
+    """Penalised rows without a top-k whose windows are taken on the device
+    (the history's hits counted per block of ids there), from an empty history
+    on, through two compactions: sample then push, both in one call
+    (run_commit), and that captured and replayed. One row without penalties
+    beside them, whose values come from the same passes."""
+    import torch
+    dev = torch.device("cuda:0")
+    B, V, W = 4, 6145, 48
+    stride, keep = 2 * W, W
+    rng = np.random.default_rng({"run": 31, "commit": 32, "captured": 33}[mode])
+    base = rng.normal(0.0, 1.0, (B, V)).astype(np.float32)
+    # the penalties decide among a few ids, at the blocks' edges and elsewhere
+    base[:, [0, 511, 512, 2047, 2048, 4095, 4096, V - 1, 77, 3000]] += 7.0
+    params = [O.identity_params(temperature=0.9, top_p=0.9, rep_penalty=1.3, repeat_last_n=W, frequency_penalty=0.4),
+              O.identity_params(temperature=1.1, min_p=0.02, rep_penalty=1.2, repeat_last_n=20, dry_multiplier=0.8,
+                                dry_base=1.75, dry_allowed_len=2, dry_last_n=W, presence_penalty=0.1),
+              O.identity_params(temperature=0.8, rep_penalty=1.5, repeat_last_n=W),
+              O.identity_params(temperature=0.8, top_p=0.95, min_p=0.05)]
+    hist = torch.zeros((B, stride), dtype=torch.int32, device=dev)
+    lens = torch.zeros(B, dtype=torch.int32, device=dev)
+    active = torch.ones(B, dtype=torch.int32, device=dev)
+    host = [[] for _ in range(B)]
+    x_d = torch.empty((B, V), dtype=torch.float32, device=dev)
+    u_d = torch.empty(B, dtype=torch.float64, device=dev)
+    stream = torch.cuda.Stream(dev)
+    out = graph = None
+
+    def step():
+        nonlocal out
+        if mode == "run":
+            out = sampler.run(x_d, params, u_d, hist=hist, hist_len=[0] * B, hist_len_dev=lens, outputs=out, stream=stream)
+            hs.history_push(hist, lens, out["token"], keep, stream=stream)
+        else:
+            out = sampler.run_commit(x_d, params, u_d, hist, [0] * B, lens, active, keep, outputs=out, stream=stream)
+
+    for s in range(2 * stride + 10):
+        x, u = _step_inputs(rng, base)
+        x_d.copy_(torch.from_numpy(x))
+        u_d.copy_(torch.from_numpy(u))
+        torch.cuda.synchronize()
+        if mode == "captured" and s == 1:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                step()
+            stream.synchronize()
+        if graph is not None:
+            graph.replay()
+        else:
+            with torch.cuda.stream(stream):
+                step()
+        torch.cuda.synchronize()
+        tok, fl = out["token"].cpu().numpy(), out["row_flags"].cpu().numpy()
+        for r in range(B):
+            _check_token(int(tok[r]), int(fl[r]), x[r], params[r], host[r], u[r], f"step {s} row {r}")
+            host[r].append(int(tok[r]))
+    got_len, got = lens.cpu().numpy(), hist.cpu().numpy()
+    for r in range(B):
+        n = int(got_len[r])
+        assert keep < n <= stride
+        np.testing.assert_array_equal(got[r, :n], host[r][-n:])
