@@ -119,6 +119,29 @@ def test_writeback_on_the_exact_lists(hs, sampler, wl, kind, kernel_mode):
     compare_rows(w, g, writeback=True)
 
 
+@pytest.mark.parametrize("k", [40, 1000])
+def test_writeback_with_penalty_tables_too_large_for_lds(hs, sampler, wl, k, kernel_mode):
+    """2048-id windows beside 250 biased ids a row, whose table the general
+    merge would keep in global memory: the exact lists take them with the
+    write-back too, which counts the history itself."""
+    from gpu_helpers import to_device
+    rng = np.random.default_rng(k)
+    B, V, L = 3, 20011, 2048
+    x = rng.normal(0, 2, size=(B, V)).astype(np.float32)
+    hist = rng.integers(0, V, (B, L)).astype(np.int32)
+    hist[1, ::2] = np.argsort(-x[1])[: L // 2]
+    plist = [wl.identity_params(temperature=0.8, top_k=k, top_p=0.95, rep_penalty=1.2, repeat_last_n=L),
+             wl.identity_params(temperature=1.1, top_k=k, frequency_penalty=0.2, presence_penalty=0.1, repeat_last_n=L),
+             wl.identity_params(temperature=0.0, rep_penalty=1.3, repeat_last_n=L)]
+    bias = [{int(t): float(v) for t, v in zip(rng.choice(V, 250, replace=False), rng.normal(-1, 2, 250))} for _ in range(B)]
+    w = _wl_from(wl, x, plist, rng.random(B), hist=hist)
+    if kernel_mode == "default":
+        xd, u, h, m = to_device(w)
+        assert sampler.query_kernels(xd, w.params, u, hist=h, hist_len=w.hist_len, bias=bias, writeback=True) & hs.KERNELS_EXACT
+    g = run_gpu(sampler, w, bias=bias, writeback=True)
+    assert compare_rows(w, g, bias=bias, writeback=True) == B
+
+
 def test_repeated_launches_are_stable(sampler, wl):
     w = wl.config(2, seed=2, rows=16)
     first = run_gpu(sampler, w)["token"]

@@ -538,9 +538,6 @@ int plan_run(const DevCaps& dc, const ultima_hsamp_batch* b, const Built& bl, Ru
         if (rp.lds_ex + statik > dc.lds_limit || pick_lds + statik > dc.lds_limit) exact = false;
         else merge_lds = pick_lds;
     }
-    // (write-back of rows whose penalty tables are too large for LDS stays with
-    // the general kernels)
-    if (rp.wb && gtab) exact = false;
     rp.exact = exact;
     rp.merge_lds = merge_lds;
     // scratch
