@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256, 2) void k_head_mm(const void* __restrict__ wei
     const int m0 = (blockIdx.x * 4 + wave) * 16;
     const int b0 = blockIdx.y * 16 * NT;
     const int H8 = H / 8 * 8;
-    const int nC = (H8 + KC - 1) / KC;
+    const int nC = H8 / KC + (H8 % KC != 0);
     const unsigned char* wrow = static_cast<const unsigned char*>(weight) + (int64_t)min(m0 + i, V - 1) * H * ES;
     // the lane's place among the LC columns: bf16, step q of four; f32, half
     // q >> 1 of step q & 1 of two
@@ -86,15 +86,17 @@ __global__ __launch_bounds__(256, 2) void k_head_mm(const void* __restrict__ wei
 
     // Addresses clamped into the rows: columns past H8 feed steps that are
     // skipped, rows past V and past the batch feed outputs that are not stored.
-    auto load_w = [&](int col) {
-        col = min(col + lcol, H8 - 16 / ES);
+    // (columns are unsigned: those past the row's end may pass 2^31)
+    auto load_w = [&](uint32_t col) {
+        col = min(col + (uint32_t)lcol, (uint32_t)(H8 - 16 / ES));
         return (u32x4)*reinterpret_cast<const u32x4_a2*>(wrow + (int64_t)col * ES);
     };
     auto load_x = [&](f32x4_a4 (&v)[NX], int c) {
 #pragma unroll
         for (int t = 0; t < NX; ++t) {
             const int n = tid + 256 * t, j = n / (KC / 4), k = n % (KC / 4) * 4;
-            v[t] = *reinterpret_cast<const f32x4_a4*>(x + (int64_t)min(b0 + j, rows - 1) * H + min(c * KC + k, H8 - 4));
+            v[t] = *reinterpret_cast<const f32x4_a4*>(x + (int64_t)min(b0 + j, rows - 1) * H +
+                                                      min((uint32_t)c * KC + k, (uint32_t)H8 - 4u));
         }
     };
     auto store_x = [&](const f32x4_a4 (&v)[NX], int buf) {
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(256, 2) void k_head_mm(const void* __restrict__ wei
         u32x4 next[NL];
         load_x(xv, min(c + 1, nC - 1));
 #pragma unroll
-        for (int t = 0; t < NL; ++t) next[t] = load_w((c + 1) * KC + t * LC);
+        for (int t = 0; t < NL; ++t) next[t] = load_w((uint32_t)(c + 1) * KC + t * LC);
         // the loads stay here, a chunk ahead of their use (the compiler moves
         // them down to it otherwise)
         __builtin_amdgcn_sched_barrier(0);
@@ -178,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void k_head_mm(const void* __restrict__ wei
     const int left = (H8 - whole * KC) >> 3;
     for (int n = 0; n < left; n += GS) {
         float a0[GS], a1[GS];
-        weights(load_w(whole * KC + 8 * n), a0, a1);
+        weights(load_w((uint32_t)whole * KC + 8 * n), a0, a1);
 #pragma unroll
         for (int s = 0; s < GS; ++s)
             if (n + s < left) step(xl[whole & 1] + xlane + 8 * (n + s), a0[s], a1[s]);

@@ -879,15 +879,16 @@ __global__ __launch_bounds__(kPrepThreads) void k_head_prep(const float* __restr
     const bool fold = fold_block > 0 && H % fold_block == 0;
     // a piece's elements, scales and signs; indices clamped into the row
     float pv[kPrepPer], sv[kPrepPer], gv[kPrepPer];
-    auto load = [&](int p0, float* v, const float* from) {
+    // (piece starts are unsigned: the one past the row's end may pass 2^31)
+    auto load = [&](uint32_t p0, float* v, const float* from) {
 #pragma unroll
-        for (int e = 0; e < kPrepPer; ++e) v[e] = from[min(p0 + tid + e * kPrepThreads, H - 1)];
+        for (int e = 0; e < kPrepPer; ++e) v[e] = from[min(p0 + tid + e * kPrepThreads, (uint32_t)H - 1u)];
     };
     load(0, pv, x);
     load(0, sv, scale);
     if (fold && signs != nullptr) load(0, gv, signs);
     float p = 0.0f;
-    for (int p0 = 0; p0 < H8; p0 += kPrepPiece) {
+    for (uint32_t p0 = 0; p0 < (uint32_t)H8; p0 += kPrepPiece) {
         if (p0 > 0) {
             load(p0, pv, x);
             __syncthreads();                                 // the previous piece's chains are done
@@ -899,7 +900,7 @@ __global__ __launch_bounds__(kPrepThreads) void k_head_prep(const float* __restr
         }
         __syncthreads();
         if (tid < 8) {
-            const int n = min(kPrepPiece, H8 - p0) >> 3;     // steps of this piece
+            const int n = min(kPrepPiece, H8 - (int)p0) >> 3;   // steps of this piece
             const float* cf = buf + tid * kPrepChain;
             const float4* cs = reinterpret_cast<const float4*>(cf);
             const int ng = n >> 4;
@@ -938,13 +939,13 @@ __global__ __launch_bounds__(kPrepThreads) void k_head_prep(const float* __restr
     }
     const float inv = 1.0f / sqrtf(ss / (float)H + eps);
     const float finv = 1.0f / sqrtf((float)fold_block);
-    for (int p0 = 0; p0 < H; p0 += kPrepPiece) {
+    for (uint32_t p0 = 0; p0 < (uint32_t)H; p0 += kPrepPiece) {
         if (H > kPrepPiece) {                                // (one piece: still in registers)
             load(p0, pv, x);
             load(p0, sv, scale);
             if (fold && signs != nullptr) load(p0, gv, signs);
         }
-        const int n = min(kPrepPiece, H - p0);
+        const int n = min(kPrepPiece, H - (int)p0);
         if (!fold) {
 #pragma unroll
             for (int e = 0; e < kPrepPer; ++e) {
