@@ -614,9 +614,11 @@ int launch_run(const RunPlan& rp, const Built& bl, const ultima_hsamp_batch* b, 
     a.fullp = buf.fullp;
     a.fs_tab = buf.fs_tab;
     // Without the copy of the transformed row, 4 bytes an id of writes: 256 rows
-    // of V = 151936, top-p: 376 us a step against 386. Rows with penalties keep it
-    // (their values are made once), those without top-p and min-p too (one row's
-    // latency: the draw reads it), and misaligned ones (element loads twice).
+    // of V = 151936, top-p: 375 us a step against 384. k_full takes what it needs
+    // from the numerators and the first pass's tables, single ids from the logits.
+    // Rows with penalties keep the copy (their values are made once), those
+    // without top-p and min-p too (one row's latency: the draw reads it), and
+    // misaligned ones (element loads twice).
     a.fs_lazy = bl.any_fpre_tp && !bl.any_fpre_plain && !bl.any_fpre_pen && rp.vec && rp.V >= 8 ? 1 : 0;
     a.wb_out = bl.any_full ? nullptr : buf.wb_out;   // (k_full writes its row back in place)
     a.full_stride = rp.full_stride;

@@ -7,8 +7,11 @@
 // rounded once to nearest, subnormals kept: the same bits as the chain's step.
 // v_mfma_f32_16x16x1_4b runs four independent 16 x 16 blocks, so two of them
 // are one step of all eight chains of a tile of 16 vocabulary rows x 16 batch
-// rows, at twice the rate of v_fma_f32 (134 against 66 TFLOP/s measured), and
-// the weights are read once per 64 batch rows instead of once per four.
+// rows. Its peak is little above v_fma_f32's (142 against 135 TFLOP/s measured
+// on independent chains), but one instruction takes 1024 multiply-adds from
+// two registers a lane where the vector form issues sixteen, each with its
+// operand read from LDS, and the accumulators of 16 x 16 outputs let the
+// weights be read once per 64 batch rows instead of once per four.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -53,8 +56,9 @@ __device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
 // LDS (rows padded by 2 floats: the 8-byte reads of a step are conflict-free),
 // the next chunk's values and weights in flight while one is multiplied.
 //
-// Bound by the matrix pipe (0.74 busy at 64 rows) and, up to 16 rows, by the
-// weights' stream. H = 4096, V = 151936 bf16, against passes of four rows
+// Bound by the matrix pipe (busy 0.75 of the SIMDs' cycles at 64 rows, where it
+// would take 561 us at the rate above) and, up to 16 rows, by the weights'
+// stream. H = 4096, V = 151936 bf16, against passes of four rows
 // through the lane-per-row kernel: 64 rows 800 us (3200), 32 rows 460 us
 // (1650), 16 rows 305 us (877), 5 rows 300 us (455); f32, 16 rows 480 us
 // (1667). No change from two vocabulary tiles per wave, reads issued a step

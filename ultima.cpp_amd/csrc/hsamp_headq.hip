@@ -334,7 +334,8 @@ struct Tile {
         }
     }
     // With the default cache policy: a span shares its first and last 128-byte
-    // lines with the chunks before and after it, which then find them in L2.
+    // lines with the chunks before and after it, which then mostly find them in
+    // L2 (from HBM come 1.18 times the bytes with Q6_K, 1.28 with Q8_0).
     // (not G16: only the granules of the rows' spans are asked for; an offset
     // past the range makes the rest read 0 without touching memory)
     __device__ __forceinline__ void load(int c, int nb) {
@@ -607,8 +608,8 @@ __global__ __launch_bounds__(256) void k_head_q(const unsigned char* __restrict_
 // 128 accumulator registers a wave) by 4 / NC groups of sixteen vocabulary
 // rows; tile and activation are shared through LDS.
 //
-// Bound by the matrix pipe (0.45 busy) and the unpacking, which share the
-// SIMD's issue. H = 4096, V = 151936, sixteen rows, passes of four rows through
+// Bound by the matrix pipe (busy 0.48 of the SIMDs' cycles) and the unpacking,
+// which share the SIMD's issue. H = 4096, V = 151936, sixteen rows, passes of four rows through
 // the vector units -> now, us: Q4_K 935 -> 295, Q5_K 931 -> 285, Q6_K
 // 1638 -> 336, Q8_0 909 -> 350, Q4_1 975 -> 265, Q5_0 1361 -> 287; 64 rows, Q4_K
 // 3630 -> 1120. Not faster: two or four batch tiles a block, double buffers,
@@ -803,8 +804,11 @@ bool offsets_fit(int64_t rb, int rows, int V, int64_t H, int nx) {
 
 // Up to kGemvRows rows (PQ2_0, whose block sums are per batch row: any number,
 // four at a time) the vector units, which unpack each value once for all rows;
-// more the matrix cores, a tile of sixteen rows costing the same for five:
-// Q4_K, 4 rows 162 us by the first, 5 rows 295 us by the second. Hidden sizes
+// more the matrix cores, a tile of sixteen rows costing little more than five:
+// H = 4096, V = 151936, us for 4 rows by the first and 5 / 16 by the second: Q4_K
+// 148, 283 / 287, Q5_K 154, 273 / 277, Q6_K 187, 321 / 330, Q8_0 197, 336 / 339,
+// Q4_1 147, 252 / 258, Q5_0 162, 277 / 280 (five rows are two passes of the
+// first); H = 1024, V = 50257 likewise (Q4_K 25, 37 / 38). Hidden sizes
 // of 2^26 and more, whose sixteen activation rows pass 32-bit offsets, stay on
 // the vector units with as many batch rows at a time as do not.
 template <int T>

@@ -930,8 +930,8 @@ __device__ __attribute__((noinline)) void finalize_row(const StreamArgs& a, cons
             // terms the tree and the sequential sums, quotients and partial
             // sums differ by < 1e-12); otherwise the reference's sequential
             // sums on one thread, ~65 us for 1000 ids: with the margin at 2e-6
-            // one or two rows of a 1024-row batch took it and the batch waited
-            // for them (k_pick_l 121 us instead of 78).
+            // a 1024-row batch that held such a row waited for it (k_pick_l 121 us
+            // instead of 78; one that holds none is as fast either way).
             bool decided = false;
             if (single || !(u > 0.0)) {
                 if (tid == 0) {
