@@ -4285,7 +4285,7 @@ __device__ __forceinline__ float plain_value(float x, bool allowed, float inv_te
 // Penalties and logit bias (PEN: some row has them) by range_penalties over a
 // block's four windows, 2048 ids at a time: bound by the reads of the history
 // by each of the row's blocks (L2) and its barriers, 11 us for 16 rows of
-// V = 151936 with 600 ids; the step 205 us against 654 for one block per row
+// V = 151936 with 600 ids; the step 199 us against 654 for one block per row
 // that probed a hash table per logit.
 // ROW: a row's windows in blocks of its own, the row the block's (always with
 // PEN); else the batch's windows in turn, the row each wave's. With the row the
